@@ -27,9 +27,16 @@ namespace oxh {
 // l, l + K, ... of i's close sublist, then of its far sublist, and the n3 /
 // n5 bonded pairs go to lanes 0 / 1.  Partial sums are combined by a fixed
 // butterfly of wave shuffles, so results do not depend on timing.  PACK
-// (K >= 2): workgroups of PACK_BS threads evaluate HB, CRST and CXST from
-// LDS work lists (the packed form in particle_forces); same results bit
-// for bit.
+// (K >= 2): workgroups of PACK_BS threads evaluate HB and CRST from an LDS
+// work list, and with K >= 4 their bonds by whole waves (the packed form in
+// particle_forces); same results bit for bit.
+// Bound by VALU issue (half of the issue slots) and the latency of each
+// round's dependent gathers and barriers, not by memory.  Pairs enter the
+// list only when every cosine of a term is inside its window
+// (hydro_active), HB and CRST items go to different waves, and a round has
+// two barriers: 24,576-nt gas (K = 8, far pairs inline) 25.3 -> 18.1 us a
+// launch, 196,608-nt bundle with its far kernel (K = 2) 269 -> 233 us,
+// all-FP64 in place 53,352-nt bundle 262 -> 213 us.
 template<int K, bool SPLIT, bool FAR, bool PACK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_forces(int N, const double4 *__restrict__ pos, const double4 *__restrict__ q64,
 		const float4 *__restrict__ q32,
@@ -55,7 +62,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 		}
 		const bool act = i < N && !idle(i, systems[s], s, k, limit);
 		particle_forces<SPLIT, FAR, true>(K, ic, l, N, pos, q64, q32, bpos, bonds, pinfo, nbr, nnbr, max_neigh, systems, sstate, Fout, Tout,
-				esplit, hbcount, stress, act, &sh);
+				esplit, hbcount, stress, act, &sh, blk * (PACK_BS / K), k, limit);
 	}
 	else {
 		if(i >= N) return;

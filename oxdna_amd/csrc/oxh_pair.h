@@ -9,20 +9,28 @@
 
 namespace oxh {
 
-// Work lists of the packed form of k_forces (one per workgroup of
-// PACK_BS threads, in LDS): the pairs of one round whose base-base
-// separation reaches HB or CRST (h) and those whose stack-stack separation
-// reaches CXST (c), one item per slot, fields as separate arrays so that
-// consecutive slots are conflict-free.  Fields of h: p's a1, a3, q's a1, a3,
-// p's base offset, base-base separation (18 floats), p's and q's base type
-// and the system (ints).  Fields of c: p's a1, a3, q's a1, a3, p's stack
-// offset, stack-stack separation.  Evaluating an item overwrites its first
-// fields with the results: force on q, lab torque on p, energies.
-constexpr int PACK_H = 21, PACK_C = 18;
+// Work list of the packed form of k_forces (one per workgroup of PACK_BS
+// threads, in LDS): the pairs of one round on which HB or CRST can act, one
+// item per slot, those with HB from the front and those with CRST alone from
+// the back, fields as separate arrays so that consecutive slots are
+// conflict-free.  Fields: p's a1, a3, q's a1, a3, p's base offset, base-base
+// separation (18 floats), p's and q's base type, the system and the terms
+// (hydro_active's flags; ints).  res: an item's results: force on q, lab
+// torque on p, energies (read while faster waves already list the next
+// round's items, hence apart from the fields).  n: items of the two kinds
+// (two sets, used by rounds in turn).  bond: both bonds of
+// the workgroup's particles (force, torque, energy), with four or more
+// lanes per nucleotide.  c: CXST results of each thread's pairs.  41 KB:
+// three workgroups per CU, as many as the registers allow.  Two entries per
+// lane and round (PACK_U = 2) measured slower (spilled registers and twice
+// the code): 242 against 237 us on the 196,608-nt bundle.
+constexpr int PACK_H = 22, PACK_U = 1, PACK_N = PACK_U * PACK_BS, PACK_BONDS = PACK_BS / 2;
 struct PackShared {
-	float h[PACK_H][PACK_BS];
-	float c[PACK_C][PACK_BS];
-	int nh[PACK_BS / 64], nc[PACK_BS / 64], rounds[PACK_BS / 64];
+	float h[PACK_H][PACK_N];
+	float res[8][PACK_N];
+	float c[7][PACK_N];
+	float bond[7][PACK_BONDS];
+	int n[2][2], rounds[PACK_BS / 64];
 };
 
 // a nucleotide's FP64 a1 axis and backbone offset (the stacking and base
@@ -39,6 +47,15 @@ __device__ __forceinline__ void sites_d(double4 q, Sites64 &st) {
 	const double b1 = (double) POS_MM_BACK1, b2 = (double) POS_MM_BACK2;
 	st.a1 = a1;
 	st.back = {b1 * a1.x + b2 * a2.x, b1 * a1.y + b2 * a2.y, b1 * a1.z + b2 * a2.z};
+}
+
+// 1 / sqrt(x) of x > 0 in FP64: the hardware's approximation (relative error
+// below 2^-20) and one cubic Newton step.  The sines of the angular factors
+// go through it in both forms (the FP32 form rounds them afterwards).
+__device__ __forceinline__ double inv_sqrt(double x) {
+	const double y = __builtin_amdgcn_rsq(x);
+	const double e = fma(-(x * y), y, 1.);
+	return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
 namespace sp {
