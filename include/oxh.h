@@ -161,7 +161,8 @@ oxh_status oxh_batch_compute_forces(oxh_batch *b);
  * reference's CUDABaseList::update when _d_are_lists_old,
  * src/CUDA/Backends/MD_CUDABackend.cu:580-590).  stream: a hipStream_t, or
  * NULL for the batch's own; the additions are queued on it (the call
- * returns after the list check, before they finish). */
+ * returns after the list check; after a rebuild the additions may still
+ * run). */
 oxh_status oxh_interaction_compute_forces(oxh_batch *b, const double *d_pos, const double *d_quat, void *d_forces, void *d_torques,
 		void *stream);
 
@@ -175,17 +176,17 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *b, const double *d_pos, con
  * Nothing is allocated: the Verlet list (built afresh on every call, all
  * pairs), the FP32 mirror, F, T and the parameters live in a fixed device
  * array of the library, OXH_NOALLOC_SCRATCH_BYTES on each GPU it runs on,
- * held until the process ends.  Limits: at most OXH_NOALLOC_MAX_N
+ * held until the process ends, and one page-locked host block that the
+ * first call allocates.  Limits: at most OXH_NOALLOC_MAX_N
  * nucleotides (larger N is rejected with OXH_ERR_ARG before any GPU work)
  * and OXH_NOALLOC_MAX_NEIGH Verlet neighbours per nucleotide (more returns
- * OXH_ERR_SYSTEM and adds nothing).  The call waits for the list and force
- * kernels, then queues the additions on `stream` (NULL: the null stream)
- * and returns.  Every call on a GPU shares that GPU's array: calls that
+ * OXH_ERR_SYSTEM and adds nothing).  The call queues its kernels on
+ * `stream` (NULL: the null stream) and returns when they have run.  Every call on a GPU shares that GPU's array: calls that
  * overlap on one GPU (other threads, other streams, a call issued before
  * the previous call's additions have run) race; serialise them. */
 #define OXH_NOALLOC_MAX_N 4096
 #define OXH_NOALLOC_MAX_NEIGH 256
-#define OXH_NOALLOC_SCRATCH_BYTES 5425408
+#define OXH_NOALLOC_SCRATCH_BYTES 5359872
 oxh_status oxh_interaction_compute_forces_noalloc(int device, const oxh_system_desc *desc, const double *d_pos, const double *d_quat,
 		void *d_forces, void *d_torques, void *stream);
 

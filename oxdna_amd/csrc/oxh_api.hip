@@ -60,6 +60,9 @@ struct oxh_batch {
 	std::vector<long long> target, done_steps;
 	double4 *bk_rlist = nullptr;
 	float4 *bk_blist = nullptr;
+	// page-locked word that a kernel writes for the host: the rebuild flag
+	// of a force call on the caller's buffers
+	int *h_flag = nullptr;
 	// external forces of each system: (particle, record) in the caller's
 	// order
 	std::vector<std::vector<std::pair<int, oxh_ext_rec>>> ext_of;
@@ -1139,6 +1142,7 @@ oxh_status oxh_batch_destroy(oxh_batch *B) {
 			b.ext_grp, b.ext_grp_sys, b.ext_idx, b.ext_com, b.blist, B->bk_blist};
 	for(void *p : ptrs)
 		if(p) (void) hipFree(p);
+	if(B->h_flag) (void) hipHostFree(B->h_flag);
 	if(b.stream) (void) hipStreamDestroy(b.stream);
 	delete B;
 	return OXH_OK;
@@ -1426,6 +1430,7 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 		if(any && !up(b.d_sys, b.h_sys.data(), n_sys * sizeof(oxh_sys))) return bail(fail(OXH_ERR_HIP, "system upload failed"));
 	}
 	TRYB(dalloc(B, &B->bk_rlist, N));
+	if(hipHostMalloc((void **) &B->h_flag, sizeof(int), hipHostMallocPortable) != hipSuccess) return bail(fail(OXH_ERR_ALLOC, "page-locked allocation failed"));
 	TRYB(dalloc(B, &b.any_rebuild, 1));
 	if(hipMemsetAsync(b.any_rebuild, 0, sizeof(int), st) != hipSuccess) return bail(fail(OXH_ERR_HIP, "memset failed"));
 	if(B->pool) TRYB(dalloc(B, &b.limit, n_sys));
@@ -1435,7 +1440,8 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 		s = autotune_forces(B);
 		if(s != OXH_OK) return bail(s);
 	}
-	else if(const char *env = getenv("OXH_FORCE_LANES")) {
+	else b.force_block = 64;   // a pool's waves seldom fill the chip: one per workgroup spreads them over more CUs
+	if(const char *env = B->pool ? getenv("OXH_FORCE_LANES") : nullptr) {
 		b.lanes = atoi(env);
 		b.far_lanes = 0;
 		if(const char *f = getenv("OXH_FAR_LANES")) b.far_lanes = atoi(f);
@@ -1517,12 +1523,21 @@ __global__ void k_load_caller_state(int N, const double4 *__restrict__ upos, con
 }
 
 // caller's F / T (upload order) += the batch's forces and torques, .w
-// included (energy share, HB energy share)
+// included (energy share, HB energy share).  Nothing is added when *hold is
+// set (lists due for a rebuild) or *err has a bit of errmask (a row that
+// overflowed); the two words go to the host's page-locked out (one word),
+// which spares the call a copy back.
 template<class FT>
 __global__ void k_add_to_caller(int N, const FT *__restrict__ F, const FT *__restrict__ T, const int *__restrict__ orig,
-		const int2 *__restrict__ pinfo, const oxh_sys *__restrict__ systems, FT *__restrict__ uF, FT *__restrict__ uT) {
+		const int2 *__restrict__ pinfo, const oxh_sys *__restrict__ systems, FT *__restrict__ uF, FT *__restrict__ uT,
+		const int *__restrict__ hold, const int *__restrict__ err, int errmask, volatile int *out) {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if(i >= N) return;
+	const int stop = (hold ? *hold : 0) | (err ? *err & errmask : 0);
+	if(i == 0 && out) {
+		*out = stop;
+		__threadfence_system();
+	}
+	if(i >= N || stop) return;
 	const oxh_sys &S = systems[pinfo[i].y];
 	if(oxh::padding(i, S)) return;
 	const int u = S.first + orig[i];
@@ -1542,6 +1557,16 @@ __global__ void k_add_to_caller(int N, const FT *__restrict__ F, const FT *__res
 	uT[u] = b;
 }
 
+void launch_add(const oxh::Batch &b, hipStream_t st, void *d_forces, void *d_torques, const int *hold, const int *err, int errmask, int *out) {
+	const int bs = 256, g = (b.N + bs - 1) / bs;
+	if(b.fp64)
+		k_add_to_caller<double4><<<g, bs, 0, st>>>(b.N, b.F64, b.T64, b.orig, b.pinfo, b.d_sys, (double4 *) d_forces, (double4 *) d_torques,
+				hold, err, errmask, out);
+	else
+		k_add_to_caller<float4><<<g, bs, 0, st>>>(b.N, b.F, b.T, b.orig, b.pinfo, b.d_sys, (float4 *) d_forces, (float4 *) d_torques, hold,
+				err, errmask, out);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1558,6 +1583,21 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *B, const double *d_pos, con
 	const int bs = 256, g = (b.N + bs - 1) / bs;
 	k_load_caller_state<<<g, bs, 0, st>>>(b.N, (const double4 *) d_pos, (const double4 *) d_quat, b.orig, b.pinfo, b.bonds, b.d_sys,
 			b.rlist, b.pos, b.q64, b.q32, b.bpos, b.back64, b.d_state, b.any_rebuild, b.blist);
+	// Most calls need no list: the forces and the additions follow at once,
+	// on the lists in hand, and both do nothing when the state just loaded
+	// asks for a rebuild.  The host learns which from the additions' word,
+	// so that a call is the state, the forces, the additions and one wait
+	// (24,576-nt gas: 106 us with the list kernels and a copy back queued in
+	// every call, 51 us without).
+	auto forces = [&](int k) {
+		if(B->persist) oxh::launch_persist_forces(st, b, false, B->persist_block);
+		else oxh::launch_forces(st, b, false, k);
+	};
+	forces(oxh::K_IF_LISTS_HOLD);
+	launch_add(b, st, d_forces, d_torques, b.any_rebuild, nullptr, 0, B->h_flag);
+	HIPCHK(hipGetLastError());
+	HIPCHK(hipStreamSynchronize(st));
+	if(*(volatile int *) B->h_flag == 0) return OXH_OK;
 	std::vector<oxh_sys_state> sst(b.nsys);
 	for(int attempt = 0;; attempt++) {
 		if(attempt == 12) return fail(OXH_ERR_SYSTEM, "neighbour list keeps overflowing");
@@ -1565,8 +1605,7 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *B, const double *d_pos, con
 		// (every system after a capacity change), then the forces
 		oxh::launch_cells(st, b, b.pos);
 		oxh::launch_build_list(st, b, 0, b.pos);
-		if(B->persist) oxh::launch_persist_forces(st, b, false, B->persist_block);
-		else oxh::launch_forces(st, b, false);
+		forces(-1);
 		HIPCHK(hipMemcpyAsync(sst.data(), b.d_state, sizeof(oxh_sys_state) * b.nsys, hipMemcpyDeviceToHost, st));
 		HIPCHK(hipStreamSynchronize(st));
 		HIPCHK(hipGetLastError());
@@ -1581,10 +1620,7 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *B, const double *d_pos, con
 		HIPCHK(hipStreamSynchronize(b.stream));
 		k_clear_need<<<(b.nsys + 63) / 64, 64, 0, st>>>(b.nsys, b.d_state, 1, b.any_rebuild);
 	}
-	if(b.fp64)
-		k_add_to_caller<double4><<<g, bs, 0, st>>>(b.N, b.F64, b.T64, b.orig, b.pinfo, b.d_sys, (double4 *) d_forces, (double4 *) d_torques);
-	else
-		k_add_to_caller<float4><<<g, bs, 0, st>>>(b.N, b.F, b.T, b.orig, b.pinfo, b.d_sys, (float4 *) d_forces, (float4 *) d_torques);
+	launch_add(b, st, d_forces, d_torques, nullptr, nullptr, 0, nullptr);
 	HIPCHK(hipGetLastError());
 	return OXH_OK;
 }
@@ -2869,7 +2905,7 @@ extern "C" oxh_status oxh_copy_bench(int device, long long bytes, int reps, doub
 // buffer beyond the caller's inputs and outputs in `scratch`, a fixed device
 // array of this library (one copy per GPU, held until the process ends).
 // Its regions, each 256-byte aligned: the system's parameters and state
-// word, the rebuild flag, the topology staging, the FP64 state and list
+// word, the rebuild flag, the FP64 state and list
 // positions, the FP32 mirror, F / T in both precisions, bonds, particle
 // info, original indices and the Verlet list (OXH_NOALLOC_MAX_NEIGH
 // entries per particle).  Host code takes its address per device from
@@ -2885,8 +2921,7 @@ struct NaLayout {
 	static constexpr size_t sys = 0;
 	static constexpr size_t state = na_up(sys + sizeof(oxh_sys));
 	static constexpr size_t any = na_up(state + sizeof(oxh_sys_state));
-	static constexpr size_t topo = na_up(any + sizeof(int));
-	static constexpr size_t pos = na_up(topo + NA_N * sizeof(int4));
+	static constexpr size_t pos = na_up(any + sizeof(int));
 	static constexpr size_t q64 = pos + NA_N * sizeof(double4);
 	static constexpr size_t rlist = q64 + NA_N * sizeof(double4);
 	static constexpr size_t back64 = rlist + NA_N * sizeof(double4);
@@ -2910,9 +2945,14 @@ static __device__ __align__(256) unsigned char scratch[NaLayout::end];
 constexpr int NA_MAX_DEVICES = 64;
 std::mutex g_na_mutex;
 unsigned char *g_na_ptr[NA_MAX_DEVICES] = {};
-// host staging of the topology (n3, n5, btype) and of the state word read back
-int4 g_na_topo[NA_N];
-oxh_sys_state g_na_state;
+// page-locked host memory, allocated by the first call and held: the
+// topology (n3, n5, btype), which the load kernel reads in place, and the
+// state word that the additions write back
+struct NaHost {
+	int4 topo[NA_N];
+	int error;
+};
+NaHost *g_na_host = nullptr;
 
 // the device address of `scratch` on `device` (current), looked up once
 oxh_status na_scratch(int device, unsigned char **out) {
@@ -2980,8 +3020,8 @@ extern "C" oxh_status oxh_interaction_compute_forces_noalloc(int device, const o
 	unsigned char *base = nullptr;
 	TRY(na_scratch(device, &base));
 	hipStream_t st = (hipStream_t) stream;
-	for(int i = 0; i < N; i++) g_na_topo[i] = make_int4(desc->n3[i], desc->n5[i], desc->btype[i], 0);
-	HIPCHK(hipMemcpyAsync(base + NaLayout::topo, g_na_topo, (size_t) N * sizeof(int4), hipMemcpyHostToDevice, st));
+	if(!g_na_host) HIPCHK(hipHostMalloc((void **) &g_na_host, sizeof(NaHost), hipHostMallocPortable));
+	for(int i = 0; i < N; i++) g_na_host->topo[i] = make_int4(desc->n3[i], desc->n5[i], desc->btype[i], 0);
 
 	oxh::Batch b;
 	b.device = device;
@@ -3012,24 +3052,19 @@ extern "C" oxh_status oxh_interaction_compute_forces_noalloc(int device, const o
 	b.model = desc->interaction == OXH_INTERACTION_DNA2 ? 0 : 1;
 	b.lanes = 8;
 	b.far_lanes = 0;
-	b.force_block = 256;
+	b.force_block = 64;   // at most 512 waves: one per workgroup, each on a CU of its own
 	b.pack = false;
 
 	const int bs = 256, g = (N + bs - 1) / bs;
-	k_na_load<<<g, bs, 0, st>>>(N, S, (const int4 *) (base + NaLayout::topo), (const double4 *) d_pos, (const double4 *) d_quat,
+	k_na_load<<<g, bs, 0, st>>>(N, S, g_na_host->topo, (const double4 *) d_pos, (const double4 *) d_quat,
 			b.d_sys, b.d_state, b.any_rebuild, b.pos, b.q64, b.q32, b.bpos, b.back64, b.bonds, b.pinfo, b.orig);
 	oxh::launch_build_list(st, b, 1, b.pos);
 	oxh::launch_forces(st, b, false);
-	HIPCHK(hipMemcpyAsync(&g_na_state, b.d_state, sizeof(oxh_sys_state), hipMemcpyDeviceToHost, st));
-	HIPCHK(hipStreamSynchronize(st));
+	launch_add(b, st, d_forces, d_torques, nullptr, &b.d_state->error, oxh::ERR_LIST, &g_na_host->error);
 	HIPCHK(hipGetLastError());
-	if(g_na_state.error & oxh::ERR_LIST)
+	HIPCHK(hipStreamSynchronize(st));
+	if(*(volatile int *) &g_na_host->error)
 		return fail(OXH_ERR_SYSTEM, "oxh_interaction_compute_forces_noalloc: a particle has more than %d neighbours (OXH_NOALLOC_MAX_NEIGH)",
 				NA_NEIGH);
-	if(b.fp64)
-		k_add_to_caller<double4><<<g, bs, 0, st>>>(N, b.F64, b.T64, b.orig, b.pinfo, b.d_sys, (double4 *) d_forces, (double4 *) d_torques);
-	else
-		k_add_to_caller<float4><<<g, bs, 0, st>>>(N, b.F, b.T, b.orig, b.pinfo, b.d_sys, (float4 *) d_forces, (float4 *) d_torques);
-	HIPCHK(hipGetLastError());
 	return OXH_OK;
 }

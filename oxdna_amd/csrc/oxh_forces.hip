@@ -49,6 +49,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 	const int t = blk * blockDim.x + threadIdx.x;
 	const int i = t / K;
 	const int l = t % K;
+	if(k == K_IF_LISTS_HOLD && *any) return;
 	if(k >= 0 && t == 0) *any = 0;   // inside a step: this step's list builds are done
 	if constexpr(PACK) {
 		// every thread of the workgroup takes part in the work lists'
@@ -346,6 +347,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
 	const int t = blk * blockDim.x + threadIdx.x;
 	const int i = t / K;
 	const int l = t % K;
+	if(k == K_IF_LISTS_HOLD && *any) return;
 	if(k >= 0 && t == 0) *any = 0;
 	if(i >= N) return;
 	const int s = pinfo[i].y;

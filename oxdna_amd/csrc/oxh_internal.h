@@ -170,6 +170,8 @@ void launch_persist_forces(hipStream_t st, const Batch &b, bool split, int block
 
 // k = index of the step inside the current chunk (checked against limit);
 // k < 0: forces of every system's current state, whatever its limit
+// (K_IF_LISTS_HOLD: nothing while *any_rebuild is set)
+constexpr int K_IF_LISTS_HOLD = -2;
 void launch_forces(hipStream_t st, const Batch &b, bool split, int k = -1);
 // list builds read positions from src (the current positions, or rlist to
 // rebuild exactly the lists of the last build)

@@ -551,6 +551,7 @@ __global__ void __launch_bounds__(64) k_forces_rna(int N, const double4 *__restr
 	const int t = blk * blockDim.x + threadIdx.x;
 	const int i = t / K;
 	const int l = t % K;
+	if(kstep == K_IF_LISTS_HOLD && *any) return;
 	if(kstep >= 0 && t == 0) *any = 0;
 	if(i >= N) return;
 	const int2 pi = pinfo[i];
