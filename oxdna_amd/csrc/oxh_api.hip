@@ -343,8 +343,15 @@ void enqueue_lists(oxh_batch *B, bool all) {
 // the chunk's start (Bussi alignment).  The second half of a step and the
 // first half of the next share one kernel, except around Bussi
 // activations, which need all of a system's velocities in between.
+void enqueue_fused(oxh_batch *B, int count, long long step_index0);
+bool fused_ok(const oxh_batch *B);
+
 void enqueue_steps(oxh_batch *B, int count, long long step_index0) {
 	oxh::Batch &b = B->b;
+	if(fused_ok(B)) {
+		enqueue_fused(B, count, step_index0);
+		return;
+	}
 	auto bussi_due = [&](int k) { return B->any_bussi && (!B->bussi_aligned || (step_index0 + k) % B->bussi_ns == 0); };
 	oxh::launch_first_step(b.stream, b, 0);   // also zeroes the cell counters
 	for(int k = 0; k < count; k++) {
@@ -356,6 +363,87 @@ void enqueue_steps(oxh_batch *B, int count, long long step_index0) {
 			oxh::launch_second_step(b.stream, b, k);
 			if(bussi_due(k)) oxh::launch_bussi(b.stream, b, k);
 			if(k + 1 < count) oxh::launch_first_step(b.stream, b, k + 1);
+		}
+	}
+}
+
+// whether the batch's steps can take one launch each (oxh_fused.hip):
+// grid-engine batches and pools of the mixed oxDNA2 form with the far pairs
+// inline and lists built per particle
+bool fused_ok(const oxh_batch *B) {
+	const oxh::Batch &b = B->b;
+	return b.fuse && !b.edge && b.far_lanes == 0 && b.n_ext == 0 && oxh::fused_lanes(b.lanes);
+}
+
+// Steps 0 .. count - 1 of a chunk, one launch each; the state is in the
+// batch's own buffers before and after.
+void enqueue_fused(oxh_batch *B, int count, long long step_index0) {
+	oxh::Batch &b = B->b;
+	auto bussi_due = [&](int k) { return B->any_bussi && (!B->bussi_aligned || (step_index0 + k) % B->bussi_ns == 0); };
+	int swaps = 0;
+	for(int k = 0; k + 1 < count; k++) swaps += !bussi_due(k);
+	const int nneed = b.nsys + 1, ncell = b.any_cells ? b.ncell_total : 0;
+	oxh::launch_step_begin(b.stream, 3 * nneed, b.step_need, 3 * ncell, b.cell_count);
+	oxh::StepArgs a = {};
+	a.N = b.N;
+	a.nsys = b.nsys;
+	a.max_neigh = b.max_neigh;
+	a.ncell = ncell;
+	a.cell_cap = b.cell_cap;
+	a.xcd = b.xcd;
+	a.vel = b.vel;
+	a.Lm = b.Lm;
+	a.rlist = b.rlist;
+	a.F = b.F;
+	a.T = b.T;
+	a.blist = b.blist;
+	a.bonds = b.bonds;
+	a.pinfo = b.pinfo;
+	a.orig = b.orig;
+	a.limit = b.limit;
+	a.pstep = b.pstep;
+	a.nbr = b.nbr;
+	a.nnbr = b.nnbr;
+	a.systems = b.d_sys;
+	a.state = b.d_state;
+	bool alt = false;   // the current state is in the other buffers
+	auto buffers = [&](bool in_alt, bool out_alt, int k) {
+		a.pos = in_alt ? b.pos_alt : b.pos;
+		a.q64 = in_alt ? b.q64_alt : b.q64;
+		a.q32 = in_alt ? b.q32_alt : b.q32;
+		a.bpos = in_alt ? b.bpos_alt : b.bpos;
+		a.pos_o = out_alt ? b.pos_alt : b.pos;
+		a.q64_o = out_alt ? b.q64_alt : b.q64;
+		a.q32_o = out_alt ? b.q32_alt : b.q32;
+		a.bpos_o = out_alt ? b.bpos_alt : b.bpos;
+		a.need = b.step_need + (k % 3) * nneed;
+		a.need_next = b.step_need + ((k + 1) % 3) * nneed;
+		a.need_clear = b.step_need + ((k + 2) % 3) * nneed;
+		a.count = b.cell_count + (size_t) (k % 3) * ncell;
+		a.count_next = b.cell_count + (size_t) ((k + 1) % 3) * ncell;
+		a.count_clear = b.cell_count + (size_t) ((k + 2) % 3) * ncell;
+		a.raw = k % 2 ? b.raw_alt : b.cell_raw;
+		a.raw_next = k % 2 ? b.cell_raw : b.raw_alt;
+		a.pos32 = k % 2 ? b.pos32_alt : b.pos32;
+		a.pos32_next = k % 2 ? b.pos32 : b.pos32_alt;
+	};
+	// an odd number of exchanges: the first half of step 0 makes one more
+	buffers(false, swaps % 2 != 0, 0);
+	oxh::launch_step_first(b.stream, a, 0);
+	alt = swaps % 2 != 0;
+	for(int k = 0; k < count; k++) {
+		const bool go_on = k + 1 < count && !bussi_due(k);
+		buffers(alt, go_on ? !alt : alt, k);
+		oxh::launch_step(b.stream, a, b.lanes, b.pack, b.force_block, k, go_on);
+		if(go_on) {
+			alt = !alt;
+			continue;
+		}
+		oxh::launch_second_step(b.stream, b, k);
+		if(bussi_due(k)) oxh::launch_bussi(b.stream, b, k);
+		if(k + 1 < count) {
+			buffers(alt, alt, k + 1);
+			oxh::launch_step_first(b.stream, a, k + 1);
 		}
 	}
 }
@@ -418,6 +506,13 @@ oxh_status alloc_cell_slots(oxh_batch *B, int cap) {
 		B->device_bytes -= 2 * ncell * b.cell_cap * sizeof(int);
 		b.cell_items = b.cell_raw = nullptr;
 	}
+	const bool two_raw = b.raw_alt != nullptr;
+	if(two_raw) {
+		HIPCHK(hipFree(b.raw_alt));
+		B->device_bytes -= ncell * b.cell_cap * sizeof(int);
+		b.raw_alt = nullptr;
+		TRY(dalloc(B, &b.raw_alt, ncell * cap));
+	}
 	b.cell_cap = cap;
 	TRY(dalloc(B, &b.cell_items, ncell * cap));
 	TRY(dalloc(B, &b.cell_raw, ncell * cap));
@@ -432,6 +527,7 @@ oxh_status grow_lists(oxh_batch *B, const std::vector<oxh_sys_state> &st) {
 	for(auto &s : st) {
 		if(s.error & oxh::ERR_LIST) grow_neigh = true;
 		if(s.error & oxh::ERR_CELLS) grow_cells = true;
+		if(s.error & oxh::ERR_ROW) b.fuse = false;
 		// a row overflow empties the row, which its partners report as well
 		if((s.error & oxh::ERR_EDGE) && !(s.error & oxh::ERR_LIST)) grow_edge = true;
 	}
@@ -1031,6 +1127,7 @@ oxh_status autotune_forces(oxh_batch *B) {
 	// 1) close kernel shape with the far pairs inline
 	b.far_lanes = 0;
 	TRY(scan_close());
+	const float inline_best = best;
 	// 2) far pairs in their own kernel, close kernel at its best shape; if
 	// that wins, the close shape again next to the far kernel
 	for(int L : lanes)
@@ -1045,6 +1142,13 @@ oxh_status autotune_forces(oxh_batch *B) {
 				bfb = bs;
 			}
 		}
+	// far pairs inline keep the step in one launch (oxh_fused.hip): their own
+	// kernel has to win by what the other launches of a step cost (four of
+	// 4 to 5 us), not by its own time alone (ms holds three evaluations)
+	if(bfl != 0 && b.fuse && inline_best <= best + 3 * 0.015f) {
+		best = inline_best;
+		bfl = 0;
+	}
 	b.far_lanes = bfl;
 	b.far_block = bfb;
 	if(bfl != 0) TRY(scan_close());
@@ -1139,7 +1243,8 @@ oxh_status oxh_batch_destroy(oxh_batch *B) {
 			b.cell_count, b.cell_items, b.cell_owner, b.pos32, b.d_sys, b.d_state, b.red_blocks, b.red_sys_blocks, b.red_partial, b.red_out, b.red_done,
 			b.esplit, b.stress, b.hbcount, b.keys, b.keys_alt, b.perm, b.perm_alt, b.inv_perm, b.radix_hist, b.scratch, B->bk_pos, B->bk_vel,
 			B->bk_Lm, B->bk_q64, B->bk_F, B->bk_T, B->bk_pstep, B->bk_state, B->bk_rlist, b.limit, b.any_rebuild, b.F64, b.T64, B->bk_F64, B->bk_T64, b.eown, b.ein, b.ecount, b.E1, b.E2, b.E3, b.B1, b.B2, b.B3, b.cell_raw, b.cell_of, b.back64, b.img, b.slot_of, b.ext_off, b.ext_rec,
-			b.ext_grp, b.ext_grp_sys, b.ext_idx, b.ext_com, b.blist, B->bk_blist};
+			b.ext_grp, b.ext_grp_sys, b.ext_idx, b.ext_com, b.blist, B->bk_blist, b.pos_alt, b.q64_alt, b.q32_alt, b.bpos_alt, b.pos32_alt,
+			b.raw_alt, b.step_need};
 	for(void *p : ptrs)
 		if(p) (void) hipFree(p);
 	if(B->h_flag) (void) hipHostFree(B->h_flag);
@@ -1269,7 +1374,7 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 	TRYB(dalloc(B, &b.pstep, N));
 	TRYB(dalloc(B, &b.nnbr, N));
 	TRYB(dalloc(B, &b.nbr, (size_t) N * b.max_neigh));
-	TRYB(dalloc(B, &b.cell_count, std::max(ncell, 1)));
+	TRYB(dalloc(B, &b.cell_count, 3 * (size_t) std::max(ncell, 1)));
 	TRYB(dalloc(B, &b.cell_owner, std::max(ncell, 1)));
 	TRYB(dalloc(B, &b.pos32, N));
 	TRYB(alloc_cell_slots(B, b.cell_cap));
@@ -1409,6 +1514,21 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 	{
 		const char *e = getenv("OXH_EDGE");
 		if(!B->pool && !B->persist && !b.fp64 && !b.model && !(e && atoi(e) == 0)) TRYB(alloc_edges(B, std::min(b.max_neigh, 64)));
+	}
+	// one launch per MD step: the second set of buffers (OXH_FUSE=0 keeps
+	// one kernel per phase)
+	{
+		const char *e = getenv("OXH_FUSE");
+		if(!B->persist && !b.fp64 && !b.model && !b.cell_build && N <= oxh::STEP_MAX_N && !(e && atoi(e) == 0)) {
+			TRYB(dalloc(B, &b.pos_alt, N));
+			TRYB(dalloc(B, &b.q64_alt, N));
+			TRYB(dalloc(B, &b.q32_alt, N));
+			TRYB(dalloc(B, &b.bpos_alt, N));
+			TRYB(dalloc(B, &b.pos32_alt, N));
+			TRYB(dalloc(B, &b.raw_alt, (size_t) std::max(ncell, 1) * b.cell_cap));
+			TRYB(dalloc(B, &b.step_need, 3 * (size_t) (n_sys + 1)));
+			b.fuse = true;
+		}
 	}
 	// far pairs kept by their backbone sites: grid-engine batches and
 	// pools, systems with cells in boxes wide enough that backbone sites

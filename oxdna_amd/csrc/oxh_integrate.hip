@@ -37,8 +37,8 @@ void launch_prepare_mirror(hipStream_t st, const Batch &b) {
 }
 
 template<class FT>
-__global__ void __launch_bounds__(256) k_first_step(int N, double4 *__restrict__ pos, double4 *__restrict__ vel, double4 *__restrict__ Lm,
-		double4 *__restrict__ q64, float4 *__restrict__ q32, float4 *__restrict__ bpos, double4 *__restrict__ back64,
+__global__ void __launch_bounds__(256) k_first_step(int N, double4 *pos, double4 *__restrict__ vel, double4 *__restrict__ Lm,
+		double4 *q64, float4 *__restrict__ q32, float4 *__restrict__ bpos, double4 *__restrict__ back64,
 		const FT *__restrict__ F, const FT *__restrict__ T, const double4 *__restrict__ rlist, const int2 *__restrict__ bonds, const int2 *__restrict__ pinfo,
 		long long *__restrict__ pstep, const oxh_sys *__restrict__ systems, oxh_sys_state *__restrict__ st, int ncell,
 		int *__restrict__ cell_count, int k, const int *__restrict__ limit, int *__restrict__ any, const float4 *__restrict__ blist) {
@@ -50,7 +50,8 @@ __global__ void __launch_bounds__(256) k_first_step(int N, double4 *__restrict__
 	const int s = pinfo[i].y;
 	const oxh_sys &S = systems[s];
 	if(idle(i, S, s, k, limit)) return;
-	if(first_step_particle(i, S, pos, vel, Lm, q64, q32, bpos, back64, F, T, rlist, bonds, pstep, blist)) {
+	double4 r;
+	if(first_step_particle(i, S, pos, vel, Lm, q64, q32, bpos, back64, F, T, rlist, bonds, pstep, blist, pos, q64, r)) {
 		st[s].need_rebuild = 1;
 		*any = 1;
 	}
@@ -95,8 +96,8 @@ void launch_second_step(hipStream_t st, const Batch &b, int k) {
 // per-particle functions in the same order as k_second_step followed by
 // k_first_step.
 template<class FT>
-__global__ void __launch_bounds__(256) k_second_first(int N, double4 *__restrict__ pos, double4 *__restrict__ vel,
-		double4 *__restrict__ Lm, double4 *__restrict__ q64, float4 *__restrict__ q32, float4 *__restrict__ bpos,
+__global__ void __launch_bounds__(256) k_second_first(int N, double4 *pos, double4 *__restrict__ vel,
+		double4 *__restrict__ Lm, double4 *q64, float4 *__restrict__ q32, float4 *__restrict__ bpos,
 		double4 *__restrict__ back64, const FT *__restrict__ F, const FT *__restrict__ T, const double4 *__restrict__ rlist,
 		const int2 *__restrict__ bonds, const int2 *__restrict__ pinfo, const int *__restrict__ orig, long long *__restrict__ pstep, const oxh_sys *__restrict__ systems,
 		oxh_sys_state *__restrict__ st, int ncell, int *__restrict__ cell_count, int k, const int *__restrict__ limit,
@@ -109,7 +110,8 @@ __global__ void __launch_bounds__(256) k_second_first(int N, double4 *__restrict
 	if(padding(i, S)) return;
 	if(!(limit && k >= limit[s])) second_step_particle(i, S, vel, Lm, F, T, orig, pstep);
 	if(!(limit && k + 1 >= limit[s])) {
-		if(first_step_particle(i, S, pos, vel, Lm, q64, q32, bpos, back64, F, T, rlist, bonds, pstep, blist)) {
+		double4 r;
+		if(first_step_particle(i, S, pos, vel, Lm, q64, q32, bpos, back64, F, T, rlist, bonds, pstep, blist, pos, q64, r)) {
 			st[s].need_rebuild = 1;
 			*any = 1;
 		}

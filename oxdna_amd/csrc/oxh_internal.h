@@ -79,6 +79,13 @@ struct Batch {
 	// in this step, cleared by the step's second half; the per-step cell and
 	// list kernels return at once while it is clear
 	int *any_rebuild = nullptr;
+	// one launch per MD step (oxh_fused.hip): the other set of state buffers,
+	// cell slots and wrapped centres; three sets of rebuild flags (one per
+	// system, then one for the batch) and of cell counters (cell_count)
+	double4 *pos_alt = nullptr, *q64_alt = nullptr;
+	float4 *q32_alt = nullptr, *bpos_alt = nullptr, *pos32_alt = nullptr;
+	int *raw_alt = nullptr, *step_need = nullptr;
+	bool fuse = false;
 
 	// reductions: blocks of at most RED_CHUNK particles, each inside one system
 	int nred = 0;
@@ -141,7 +148,8 @@ struct Batch {
 // oxh_sys_state.error bits
 constexpr int ERR_BOND = 1, ERR_LIST = 2, ERR_CELLS = 4, ERR_EDGE = 8;
 constexpr int ERR_EXT = 16;   // a particle where an external force is undefined (the reference throws)
-constexpr int ERR_OVERFLOW = ERR_LIST | ERR_CELLS | ERR_EDGE;   // fixed by growing a buffer and replaying
+constexpr int ERR_ROW = 32;   // a row longer than k_step sorts in LDS: the batch goes on with one kernel per phase
+constexpr int ERR_OVERFLOW = ERR_LIST | ERR_CELLS | ERR_EDGE | ERR_ROW;   // fixed by growing a buffer and replaying
 
 constexpr int RED_CHUNK = 2048;
 constexpr int RED_W = 8;   // reduction width: U, Uhb, Kt, Kr, vx, vy, vz, count
@@ -184,6 +192,37 @@ void launch_second_step(hipStream_t st, const Batch &b, int k);
 // second half of step k + first half of step k + 1
 void launch_second_first(hipStream_t st, const Batch &b, int k);
 void launch_bussi(hipStream_t st, const Batch &b, int k);
+
+// one launch per MD step: what k_step reads and writes at step k (buffers
+// picked by the caller; _o: the state after the step's boundary; need,
+// count, raw, pos32: of step k, _next: of step k + 1, _clear: of step k + 2)
+struct StepArgs {
+	int N, nsys, max_neigh, ncell, cell_cap, xcd;
+	const double4 *pos, *q64;
+	const float4 *q32, *bpos;
+	double4 *pos_o, *q64_o;
+	float4 *q32_o, *bpos_o;
+	double4 *vel, *Lm, *rlist;
+	float4 *F, *T, *blist;
+	const int2 *bonds, *pinfo;
+	const int *orig, *limit;
+	long long *pstep;
+	int *nbr;
+	int2 *nnbr;
+	const oxh_sys *systems;
+	oxh_sys_state *state;
+	int *need, *need_next, *need_clear;
+	int *count, *count_next, *count_clear;
+	int *raw, *raw_next;
+	float4 *pos32, *pos32_next;
+};
+// longest list row of a system with cells, and largest batch, that k_step
+// builds (a row's keys wait in LDS, (stencil cell << 24) | particle)
+constexpr int STEP_ROW = 512, STEP_MAX_N = 1 << 24;
+bool fused_lanes(int lanes);
+void launch_step_begin(hipStream_t st, int nneed, int *need, int ncount, int *count);
+void launch_step_first(hipStream_t st, const StepArgs &a, int k);
+void launch_step(hipStream_t st, const StepArgs &a, int lanes, bool pack, int block, int k, bool go_on);
 void launch_reduce(hipStream_t st, const Batch &b);
 // velocities ~ N(0, T) for particles [i0, i0 + n)
 void launch_refresh_vel(hipStream_t st, const Batch &b, int i0, int n);

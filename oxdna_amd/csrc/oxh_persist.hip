@@ -65,7 +65,8 @@ __global__ void __launch_bounds__(BLOCK) k_persist(PersistArgs a) {
 	__syncthreads();
 	for(int it = 0; it < nsteps; it++) {
 		// 1. first half kick, drift, rotation, FP32 mirror, skin check
-		if(tid < n && first_step_particle(first + tid, S, a.pos, a.vel, a.Lm, a.q64, a.q32, a.bpos, nullptr, a.F, a.T, a.rlist, a.bonds, a.pstep, nullptr))
+		double4 r;
+		if(tid < n && first_step_particle(first + tid, S, a.pos, a.vel, a.Lm, a.q64, a.q32, a.bpos, nullptr, a.F, a.T, a.rlist, a.bonds, a.pstep, nullptr, a.pos, a.q64, r))
 			need = 1;
 		__syncthreads();
 		// 2. Verlet rebuild (all pairs of the system; such systems use no cells)
@@ -198,7 +199,8 @@ __global__ void __launch_bounds__(BLOCK) k_persist_lds(PersistArgs a, int nmax) 
 	__syncthreads();
 	for(int it = 0; it < nsteps; it++) {
 		// 1. first half kick, drift, rotation, FP32 mirror, skin check
-		if(tid < n && first_step_particle(tid, S, L.pos, L.vel, L.Lm, L.q64, L.q32, L.bpos, nullptr, L.F, L.T, L.rlist, L.bonds, L.pstep, nullptr))
+		double4 r;
+		if(tid < n && first_step_particle(tid, S, L.pos, L.vel, L.Lm, L.q64, L.q32, L.bpos, nullptr, L.F, L.T, L.rlist, L.bonds, L.pstep, nullptr, L.pos, L.q64, r))
 			need = 1;
 		__syncthreads();
 		// 2. Verlet rebuild (all pairs of the system)

@@ -63,15 +63,17 @@ __device__ __forceinline__ bool back_moved(float4 b, float4 bl, const oxh_sys &S
 }
 
 // first half kick, drift and rotation of particle i, FP32 mirror, step
-// counter; returns true when the particle moved more than the skin since
+// counter; the new position (also in r) and quaternion go to pos_o and q64_o
+// (pos and q64 themselves, or another set of buffers); returns true when the particle moved more than the skin since
 // the last list build, or its backbone site more than its bound when far
 // pairs are kept by backbone sites (blist: the sites at the build; may be
 // null) (src/CUDA/Backends/CUDA_mixed.cuh:23-69)
 template<class FT>
-__device__ __forceinline__ bool first_step_particle(int i, const oxh_sys &S, double4 *__restrict__ pos, double4 *__restrict__ vel,
-		double4 *__restrict__ Lm, double4 *__restrict__ q64, float4 *__restrict__ q32, float4 *__restrict__ bpos,
+__device__ __forceinline__ bool first_step_particle(int i, const oxh_sys &S, const double4 *pos, double4 *__restrict__ vel,
+		double4 *__restrict__ Lm, const double4 *q64, float4 *__restrict__ q32, float4 *__restrict__ bpos,
 		double4 *__restrict__ back64, const FT *__restrict__ F, const FT *__restrict__ T, const double4 *__restrict__ rlist,
-		const int2 *__restrict__ bonds, long long *__restrict__ pstep, const float4 *__restrict__ blist) {
+		const int2 *__restrict__ bonds, long long *__restrict__ pstep, const float4 *__restrict__ blist, double4 *pos_o, double4 *q64_o,
+		double4 &r) {
 	const double hdt = 0.5 * S.dt;
 
 	const FT f = F[i];
@@ -80,11 +82,11 @@ __device__ __forceinline__ bool first_step_particle(int i, const oxh_sys &S, dou
 	v.y += (double) f.y * hdt;
 	v.z += (double) f.z * hdt;
 	vel[i] = v;
-	double4 r = pos[i];
+	r = pos[i];
 	r.x += v.x * S.dt;
 	r.y += v.y * S.dt;
 	r.z += v.z * S.dt;
-	pos[i] = r;
+	pos_o[i] = r;
 
 	const FT t = T[i];
 	double4 L = Lm[i];
@@ -104,8 +106,8 @@ __device__ __forceinline__ bool first_step_particle(int i, const oxh_sys &S, dou
 		q.y *= qn;
 		q.z *= qn;
 		q.w *= qn;
-		q64[i] = q;
 	}
+	q64_o[i] = q;
 	const float4 bp = write_mirror(i, r, q, S, bonds[i], q32, bpos, back64);
 	pstep[i] += 1;
 
