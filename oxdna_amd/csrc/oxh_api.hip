@@ -63,6 +63,13 @@ struct oxh_batch {
 	// page-locked word that a kernel writes for the host: the rebuild flag
 	// of a force call on the caller's buffers
 	int *h_flag = nullptr;
+	// what the host reads: page-locked staging (two halves), and the device
+	// buffer of what does not fit in STAGE_DIRECT
+	std::mutex stage_mutex;
+	unsigned char *stage = nullptr;
+	size_t stage_bytes = 0;
+	double *d_export = nullptr;
+	hipEvent_t stage_done[2] = {nullptr, nullptr};
 	// external forces of each system: (particle, record) in the caller's
 	// order
 	std::vector<std::vector<std::pair<int, oxh_ext_rec>>> ext_of;
@@ -289,17 +296,6 @@ void frame_to_quat(const double *a1, const double *a3, double q[4]) {
 	q[1] = y / n;
 	q[2] = z / n;
 	q[3] = w / n;
-}
-
-void quat_to_axes(const double4 &q, double a1[3], double a3[3]) {
-	double sqx = q.x * q.x, sqy = q.y * q.y, sqz = q.z * q.z, sqw = q.w * q.w;
-	double xy = q.x * q.y, xz = q.x * q.z, xw = q.x * q.w, yz = q.y * q.z, yw = q.y * q.w, zw = q.z * q.w;
-	a1[0] = sqx - sqy - sqz + sqw;
-	a1[1] = 2. * (xy + zw);
-	a1[2] = 2. * (xz - yw);
-	a3[0] = 2. * (xz + yw);
-	a3[1] = 2. * (yz - xw);
-	a3[2] = -sqx - sqy + sqz + sqw;
 }
 
 __global__ void k_clear_need(int nsys, oxh_sys_state *st, int set_value, int *any) {
@@ -952,6 +948,69 @@ void red_layout(const oxh_batch *B, std::vector<int3> &rb, std::vector<int2> &rs
 }  // namespace
 
 namespace {
+// Kernels write up to STAGE_DIRECT bytes straight into the page-locked
+// staging (a state of 546 nt); more goes through a device buffer and two
+// halves of at most 1 MiB, so that the host empties one while the other
+// fills.  Scattered writes of 24 bytes over the bus are slower than the
+// extra copy once there are many.
+constexpr size_t STAGE_DIRECT = 64 << 10, STAGE_MAX = 2 << 20;
+
+oxh_status alloc_stage(oxh_batch *B) {
+	size_t most = 0;
+	for(int s = 0; s < B->b.nsys; s++) most = std::max(most, (size_t) (B->pool ? B->cap[s] : B->n[s]) * 15 * sizeof(double));
+	B->stage_bytes = std::min(STAGE_MAX, std::max(std::max(most, (size_t) B->b.nsys * oxh::RED_W * sizeof(double)), (size_t) 4096));
+	if(hipHostMalloc((void **) &B->stage, B->stage_bytes, hipHostMallocPortable) != hipSuccess) return fail(OXH_ERR_ALLOC, "page-locked allocation failed");
+	if(most <= STAGE_DIRECT) return OXH_OK;
+	for(hipEvent_t &e : B->stage_done) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+	return dalloc(B, &B->d_export, most / sizeof(double));
+}
+
+struct StagePart {
+	double *to;   // may be null: not wanted
+	size_t count;
+};
+
+// what launch writes (to the address it is given), part after part, to the
+// caller's arrays
+template<class L>
+oxh_status fetch(oxh_batch *B, std::initializer_list<StagePart> parts, L &&launch) {
+	std::lock_guard<std::mutex> lock(B->stage_mutex);
+	size_t bytes = 0;
+	for(const StagePart &p : parts) bytes += p.count * sizeof(double);
+	if(bytes == 0) return sync_and_check(B);
+	// bytes [from, from + len) of the parts, which lie at src
+	auto unpack = [&](size_t from, size_t len, const unsigned char *src) {
+		size_t at = 0;
+		for(const StagePart &p : parts) {
+			const size_t n = p.count * sizeof(double), lo = std::max(at, from), hi = std::min(at + n, from + len);
+			if(p.to && lo < hi) std::memcpy((unsigned char *) p.to + (lo - at), src + (lo - from), hi - lo);
+			at += n;
+		}
+	};
+	if(bytes <= STAGE_DIRECT) {
+		launch((double *) B->stage);
+		TRY(sync_and_check(B));
+		unpack(0, bytes, B->stage);
+		return OXH_OK;
+	}
+	launch(B->d_export);
+	const size_t half = B->stage_bytes / 2;
+	const size_t turns = (bytes + half - 1) / half;
+	auto length = [&](size_t c) { return std::min(half, bytes - c * half); };
+	for(size_t c = 0; c <= turns; c++) {
+		if(c < turns) {
+			HIPCHK(hipMemcpyAsync(B->stage + (c & 1) * half, (unsigned char *) B->d_export + c * half, length(c), hipMemcpyDeviceToHost, B->b.stream));
+			HIPCHK(hipEventRecord(B->stage_done[c & 1], B->b.stream));
+		}
+		if(c == 0) continue;
+		HIPCHK(hipEventSynchronize(B->stage_done[(c - 1) & 1]));
+		unpack((c - 1) * half, length(c - 1), B->stage + ((c - 1) & 1) * half);
+	}
+	return sync_and_check(B);
+}
+}  // namespace
+
+namespace {
 template<typename T>
 oxh_status download(oxh_batch *B, std::vector<T> &out, const T *src, int first, int n) {
 	out.resize(n);
@@ -1368,6 +1427,10 @@ oxh_status oxh_batch_destroy(oxh_batch *B) {
 	for(void *p : ptrs)
 		if(p) (void) hipFree(p);
 	if(B->h_flag) (void) hipHostFree(B->h_flag);
+	if(B->stage) (void) hipHostFree(B->stage);
+	if(B->d_export) (void) hipFree(B->d_export);
+	for(hipEvent_t e : B->stage_done)
+		if(e) (void) hipEventDestroy(e);
 	if(b.stream) (void) hipStreamDestroy(b.stream);
 	delete B;
 	return OXH_OK;
@@ -1671,6 +1734,7 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 	}
 	TRYB(dalloc(B, &B->bk_rlist, N));
 	if(hipHostMalloc((void **) &B->h_flag, sizeof(int), hipHostMallocPortable) != hipSuccess) return bail(fail(OXH_ERR_ALLOC, "page-locked allocation failed"));
+	if(oxh_status r = alloc_stage(B); r != OXH_OK) return bail(r);
 	TRYB(dalloc(B, &b.any_rebuild, 1));
 	if(hipMemsetAsync(b.any_rebuild, 0, sizeof(int), st) != hipSuccess) return bail(fail(OXH_ERR_HIP, "memset failed"));
 	if(B->pool) TRYB(dalloc(B, &b.limit, n_sys));
@@ -2147,40 +2211,9 @@ oxh_status oxh_batch_sync(oxh_batch *B) {
 
 oxh_status oxh_batch_get_state(oxh_batch *B, int sys, double *pos, double *a1, double *a3, double *vel, double *L) {
 	TRY(check_sys(B, sys));
-	int f = B->first[sys], n = B->n[sys];
-	std::vector<double4> p, q, v, l;
-	std::vector<int> o;
-	TRY(download(B, p, B->b.pos, f, n));
-	TRY(download(B, q, B->b.q64, f, n));
-	TRY(download(B, v, B->b.vel, f, n));
-	TRY(download(B, l, B->b.Lm, f, n));
-	TRY(download(B, o, B->b.orig, f, n));
-	TRY(sync_and_check(B));
-	for(int k = 0; k < n; k++) {
-		int i = o[k];
-		if(pos) {
-			pos[3 * i] = p[k].x;
-			pos[3 * i + 1] = p[k].y;
-			pos[3 * i + 2] = p[k].z;
-		}
-		double x1[3], x3[3];
-		quat_to_axes(q[k], x1, x3);
-		for(int c = 0; c < 3; c++) {
-			if(a1) a1[3 * i + c] = x1[c];
-			if(a3) a3[3 * i + c] = x3[c];
-		}
-		if(vel) {
-			vel[3 * i] = v[k].x;
-			vel[3 * i + 1] = v[k].y;
-			vel[3 * i + 2] = v[k].z;
-		}
-		if(L) {
-			L[3 * i] = l[k].x;
-			L[3 * i + 1] = l[k].y;
-			L[3 * i + 2] = l[k].z;
-		}
-	}
-	return OXH_OK;
+	const int f = B->first[sys], n = B->n[sys];
+	const size_t w = 3 * (size_t) n;
+	return fetch(B, {{pos, w}, {a1, w}, {a3, w}, {vel, w}, {L, w}}, [&](double *out) { oxh::launch_export_state(B->b, f, n, out); });
 }
 
 oxh_status oxh_batch_set_external_forces(oxh_batch *B, int sys, int n, const oxh_ext_force *forces, long long step0) {
@@ -2500,40 +2533,9 @@ oxh_status oxh_batch_get_order(oxh_batch *B, int sys, int *order) {
 
 oxh_status oxh_batch_get_forces(oxh_batch *B, int sys, double *F, double *T, double *Epart) {
 	TRY(check_sys(B, sys));
-	int f = B->first[sys], n = B->n[sys];
-	std::vector<double4> hf(n), ht(n);
-	std::vector<int> o;
-	if(B->b.fp64) {
-		TRY(download(B, hf, B->b.F64, f, n));
-		TRY(download(B, ht, B->b.T64, f, n));
-	}
-	else {
-		std::vector<float4> sf, sT;
-		TRY(download(B, sf, B->b.F, f, n));
-		TRY(download(B, sT, B->b.T, f, n));
-		TRY(sync_and_check(B));
-		for(int k = 0; k < n; k++) {
-			hf[k] = make_double4(sf[k].x, sf[k].y, sf[k].z, sf[k].w);
-			ht[k] = make_double4(sT[k].x, sT[k].y, sT[k].z, sT[k].w);
-		}
-	}
-	TRY(download(B, o, B->b.orig, f, n));
-	TRY(sync_and_check(B));
-	for(int k = 0; k < n; k++) {
-		int i = o[k];
-		if(F) {
-			F[3 * i] = hf[k].x;
-			F[3 * i + 1] = hf[k].y;
-			F[3 * i + 2] = hf[k].z;
-		}
-		if(T) {
-			T[3 * i] = ht[k].x;
-			T[3 * i + 1] = ht[k].y;
-			T[3 * i + 2] = ht[k].z;
-		}
-		if(Epart) Epart[i] = hf[k].w;
-	}
-	return OXH_OK;
+	const int f = B->first[sys], n = B->n[sys];
+	const size_t w = 3 * (size_t) n;
+	return fetch(B, {{F, w}, {T, w}, {Epart, (size_t) n}}, [&](double *out) { oxh::launch_export_forces(B->b, f, n, out); });
 }
 
 oxh_status oxh_batch_pair_quantities(oxh_batch *B, int sys, int kind, int n, const int *pairs, double *out) {
@@ -2634,60 +2636,37 @@ extern "C" {
 oxh_status oxh_batch_energies(oxh_batch *B, double *out4) {
 	if(!B || !out4) return fail(OXH_ERR_ARG, "bad arguments");
 	HIPCHK(hipSetDevice(B->b.device));
-	oxh::launch_reduce(B->b.stream, B->b);
-	std::vector<double> r((size_t) B->b.nsys * oxh::RED_W);
-	HIPCHK(hipMemcpyAsync(r.data(), B->b.red_out, r.size() * sizeof(double), hipMemcpyDeviceToHost, B->b.stream));
+	const size_t count = (size_t) B->b.nsys * oxh::RED_W;
+	std::lock_guard<std::mutex> lock(B->stage_mutex);
+	std::vector<double> r;
+	const double *sums = (const double *) B->stage;
+	if(count * sizeof(double) <= B->stage_bytes) {
+		std::memset(B->stage, 0, count * sizeof(double));
+		oxh::launch_reduce(B->b.stream, B->b, (double *) B->stage);
+	}
+	else {
+		oxh::launch_reduce(B->b.stream, B->b);
+		TRY(download(B, r, B->b.red_out, 0, (int) count));
+		sums = r.data();
+	}
 	TRY(sync_and_check(B));
 	for(int s = 0; s < B->b.nsys; s++)
-		for(int k = 0; k < 4; k++) out4[4 * s + k] = r[(size_t) s * oxh::RED_W + k];
+		for(int k = 0; k < 4; k++) out4[4 * s + k] = sums[(size_t) s * oxh::RED_W + k];
 	return OXH_OK;
 }
 
 oxh_status oxh_batch_energy_split(oxh_batch *B, int sys, double *E8) {
 	TRY(check_sys(B, sys));
 	enqueue_forces(B, true);
-	int f = B->first[sys], n = B->n[sys];
-	std::vector<double> e((size_t) 8 * n);
-	for(int t = 0; t < 8; t++)
-		HIPCHK(hipMemcpyAsync(e.data() + (size_t) t * n, B->b.esplit + (size_t) t * B->b.N + f, n * sizeof(double), hipMemcpyDeviceToHost,
-				B->b.stream));
-	TRY(sync_and_check(B));
-	for(int t = 0; t < 8; t++) {
-		double acc = 0;
-		for(int k = 0; k < n; k++) acc += e[(size_t) t * n + k];
-		E8[t] = acc;
-	}
-	return OXH_OK;
+	const int f = B->first[sys], n = B->n[sys];
+	return fetch(B, {{E8, 8}}, [&](double *out) { oxh::launch_sums(B->b, n, 8, B->b.esplit + f, nullptr, out); });
 }
 
 oxh_status oxh_batch_stress(oxh_batch *B, int sys, double *virial6, double *kinetic6) {
 	TRY(check_sys(B, sys));
 	enqueue_forces(B, true);
 	const int f = B->first[sys], n = B->n[sys];
-	std::vector<double> w((size_t) 6 * std::max(n, 1));
-	for(int c = 0; c < 6; c++)
-		HIPCHK(hipMemcpyAsync(w.data() + (size_t) c * n, B->b.stress + (size_t) c * B->b.N + f, n * sizeof(double), hipMemcpyDeviceToHost,
-				B->b.stream));
-	std::vector<double4> v;
-	TRY(download(B, v, B->b.vel, f, n));
-	TRY(sync_and_check(B));
-	for(int c = 0; c < 6; c++) {
-		double acc = 0.;
-		for(int k = 0; k < n; k++) acc += w[(size_t) c * n + k];
-		if(virial6) virial6[c] = acc;
-	}
-	if(kinetic6) {
-		for(int c = 0; c < 6; c++) kinetic6[c] = 0.;
-		for(const double4 &x : v) {
-			kinetic6[0] += x.x * x.x;
-			kinetic6[1] += x.y * x.y;
-			kinetic6[2] += x.z * x.z;
-			kinetic6[3] += x.x * x.y;
-			kinetic6[4] += x.x * x.z;
-			kinetic6[5] += x.y * x.z;
-		}
-	}
-	return OXH_OK;
+	return fetch(B, {{virial6, 6}, {kinetic6, 6}}, [&](double *out) { oxh::launch_sums(B->b, n, 6, B->b.stress + f, B->b.vel + f, out); });
 }
 
 oxh_status oxh_batch_hb_count(oxh_batch *B, int *out) {
@@ -2696,12 +2675,17 @@ oxh_status oxh_batch_hb_count(oxh_batch *B, int *out) {
 	B->b.want_hbcount = true;
 	enqueue_forces(B);
 	B->b.want_hbcount = false;
-	std::vector<int> h(B->b.N);
-	HIPCHK(hipMemcpyAsync(h.data(), B->b.hbcount, B->b.N * sizeof(int), hipMemcpyDeviceToHost, B->b.stream));
+	std::lock_guard<std::mutex> lock(B->stage_mutex);
+	std::vector<int> h;
+	const long long *sums = (const long long *) B->stage;
+	const bool staged = (size_t) B->b.nsys * sizeof(long long) <= B->stage_bytes;
+	if(staged) oxh::launch_count(B->b, (long long *) B->stage);
+	else TRY(download(B, h, B->b.hbcount, 0, B->b.N));
 	TRY(sync_and_check(B));
 	for(int s = 0; s < B->b.nsys; s++) {
-		long long acc = 0;
-		for(int i = B->first[s]; i < B->first[s] + B->n[s]; i++) acc += h[i];
+		long long acc = staged ? sums[s] : 0;
+		if(!staged)
+			for(int i = B->first[s]; i < B->first[s] + B->n[s]; i++) acc += h[i];
 		out[s] = (int) (acc / 2);
 	}
 	return OXH_OK;

@@ -161,22 +161,21 @@ __global__ void __launch_bounds__(256) k_reduce_partial(const int3 *__restrict__
 	if(threadIdx.x < RED_W) partial[(size_t) blockIdx.x * RED_W + threadIdx.x] = sh[threadIdx.x][0];
 }
 
-__global__ void k_reduce_final(int nsys, const int2 *__restrict__ sys_blocks, const double *__restrict__ partial, double *__restrict__ out) {
-	int s = blockIdx.x * blockDim.x + threadIdx.x;
+// one thread per sum
+__global__ void __launch_bounds__(256) k_reduce_final(int nsys, const int2 *__restrict__ sys_blocks, const double *__restrict__ partial, double *__restrict__ out) {
+	const int s = (blockIdx.x * blockDim.x + threadIdx.x) / RED_W, k = threadIdx.x % RED_W;
 	if(s >= nsys) return;
-	int2 sb = sys_blocks[s];
-	for(int k = 0; k < RED_W; k++) {
-		double acc = 0.;
-		for(int b = sb.x; b < sb.x + sb.y; b++) acc += partial[(size_t) b * RED_W + k];
-		out[(size_t) s * RED_W + k] = acc;
-	}
+	const int2 sb = sys_blocks[s];
+	double acc = 0.;
+	for(int b = sb.x; b < sb.x + sb.y; b++) acc += partial[(size_t) b * RED_W + k];
+	out[(size_t) s * RED_W + k] = acc;
 }
 
-void launch_reduce(hipStream_t st, const Batch &b) {
+void launch_reduce(hipStream_t st, const Batch &b, double *out) {
 	if(b.nred == 0) return;
 	if(b.fp64) k_reduce_partial<<<b.nred, 256, 0, st>>>(b.red_blocks, b.F64, b.T64, b.vel, b.Lm, b.red_partial);
 	else k_reduce_partial<<<b.nred, 256, 0, st>>>(b.red_blocks, b.F, b.T, b.vel, b.Lm, b.red_partial);
-	k_reduce_final<<<(b.nsys + 63) / 64, 64, 0, st>>>(b.nsys, b.red_sys_blocks, b.red_partial, b.red_out);
+	k_reduce_final<<<(b.nsys * RED_W + 255) / 256, 256, 0, st>>>(b.nsys, b.red_sys_blocks, b.red_partial, out ? out : b.red_out);
 }
 
 // One pass over velocities and angular momenta: every block reduces its

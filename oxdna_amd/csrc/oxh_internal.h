@@ -223,7 +223,7 @@ bool fused_lanes(int lanes);
 void launch_step_begin(hipStream_t st, int nneed, int *need, int ncount, int *count);
 void launch_step_first(hipStream_t st, const StepArgs &a, int k);
 void launch_step(hipStream_t st, const StepArgs &a, int lanes, bool pack, int block, int k, bool go_on);
-void launch_reduce(hipStream_t st, const Batch &b);
+void launch_reduce(hipStream_t st, const Batch &b, double *out = nullptr);   // out: elsewhere than red_out
 // velocities ~ N(0, T) for particles [i0, i0 + n)
 void launch_refresh_vel(hipStream_t st, const Batch &b, int i0, int n);
 void launch_prepare_mirror(hipStream_t st, const Batch &b);
@@ -240,6 +240,12 @@ void launch_rna_forces(hipStream_t st, const Batch &b, bool split, int k);
 void launch_rna_pair_quantities(hipStream_t st, const Batch &b, int sys, int kind, int n, const int4 *d_pairs, double *d_out);
 // per-pair FFS order-parameter quantities (OXH_PAIR_*) of system sys:
 // pairs (p, q, same strand, unused) in the system's upload order
+// state / forces of particles first .. first + n - 1 as the caller's arrays;
+// row sums (and those of the products of vel); each system's hbcount
+void launch_export_state(const Batch &b, int first, int n, double *out);
+void launch_export_forces(const Batch &b, int first, int n, double *out);
+void launch_sums(const Batch &b, int n, int rows, const double *x, const double4 *vel, double *out);
+void launch_count(const Batch &b, long long *out);
 void launch_pair_quantities(hipStream_t st, const Batch &b, int sys, int kind, int n, const int4 *d_pairs, double *d_out);
 
 }  // namespace oxh
