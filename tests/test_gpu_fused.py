@@ -107,3 +107,19 @@ def test_rows_longer_than_the_step_kernel_sorts(hip, monkeypatch):
     with hip.HIPBatch(s) as b:
         assert b.stats()["mean_neigh"] > 512   # the case this test is for
     _agree(*got)
+
+
+@pytest.mark.parametrize("lanes", [2, 4, 16, 32])
+def test_rows_of_several_particles(hip, monkeypatch, lanes):
+    # systems that end inside a group's rows, some with cells
+    ss = [_gas(5, 1, 5), _gas(6, 1, 9), _gas(7, 3, 11), _gas(8, 33, 17), _gas(9, 7, 13)]
+    per = [dict(seed=100 + k) for k in range(len(ss))]
+    got = []
+    for fuse in (1, 0):
+        monkeypatch.setenv("OXH_FUSE", str(fuse))
+        monkeypatch.setenv("OXH_PERSIST", "0")
+        monkeypatch.setenv("OXH_FORCE_LANES", str(lanes))
+        with hip.HIPBatch(ss, options=per, dt=0.003, verlet_skin=0.05, refresh_vel=True, **THERMO["langevin"]) as b:
+            b.run(96)
+            got.append([dict(b.state(k), F=b.forces(k)[0], rebuilds=b.info(k)[0]) for k in range(len(ss))])
+    _agree(*got)
