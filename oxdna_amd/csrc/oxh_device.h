@@ -192,4 +192,13 @@ __device__ __forceinline__ bool idle(int i, const oxh_sys &S, int s, int k, cons
 	return padding(i, S) || (limit && k >= limit[s]);
 }
 
+// 1 / sqrt(x) of x > 0 in FP64: the hardware's approximation (relative error
+// below 2^-20) and one cubic Newton step.  The sines of the angular factors
+// go through it in both forms (the FP32 form rounds them afterwards).
+__device__ __forceinline__ double inv_sqrt(double x) {
+	const double y = __builtin_amdgcn_rsq(x);
+	const double e = fma(-(x * y), y, 1.);
+	return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 }  // namespace oxh

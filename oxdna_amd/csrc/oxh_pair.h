@@ -49,15 +49,6 @@ __device__ __forceinline__ void sites_d(double4 q, Sites64 &st) {
 	st.back = {b1 * a1.x + b2 * a2.x, b1 * a1.y + b2 * a2.y, b1 * a1.z + b2 * a2.z};
 }
 
-// 1 / sqrt(x) of x > 0 in FP64: the hardware's approximation (relative error
-// below 2^-20) and one cubic Newton step.  The sines of the angular factors
-// go through it in both forms (the FP32 form rounds them afterwards).
-__device__ __forceinline__ double inv_sqrt(double x) {
-	const double y = __builtin_amdgcn_rsq(x);
-	const double e = fma(-(x * y), y, 1.);
-	return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
 namespace sp {
 using real = float;
 using vec = f3;

@@ -100,9 +100,40 @@ __device__ __forceinline__ A f4(A t) {
 	return val;
 }
 
-// (df4/dtheta) / sin(theta), with the reference's guard for a small sine
+// 1 / sin(acos(c)): a square root instead of a sine and a division per
+// factor, in the all-FP64 form
+template<typename A>
+__device__ __forceinline__ A rsin(double c) { return (A) inv_sqrt(fmax((1. - c) * (1. + c), 1e-30)); }
+
+// 1 / sin(n PIf - acos(c)), n = 1 or 2, up to the sign: the model's pi is the
+// FP32 one, 8.7e-8 above pi, which an FP64 sine sees
+template<int n, typename A>
+__device__ __forceinline__ A rsin_pi(double c) {
+	const double rs = rsin<double>(c);
+	const double x = n * ((double) PIf - 3.14159265358979323846) * c * rs;
+	return (A) fma(rs * x, 1. + x, rs);
+}
+
+// Sine of an FP32 angle in [0, 3 pi / 2]: x or pi - x (exact but for the last
+// step), then the Taylor polynomial, whose rest is below 1e-9 up to pi / 2
+__device__ __forceinline__ float sin_angle(float t) {
+	const float x = t > 0.5f * PIf ? (PIf - t) - 8.74227766e-8f : t, y = x * x;
+	float p = 1.f / 6227020800.f;
+	p = fmaf(p, y, -1.f / 39916800.f);
+	p = fmaf(p, y, 1.f / 362880.f);
+	p = fmaf(p, y, -1.f / 5040.f);
+	p = fmaf(p, y, 1.f / 120.f);
+	p = fmaf(p, y, -1.f / 6.f);
+	return fmaf(p * y, x, x);
+}
+
+// (df4/dtheta) / sin(theta), with the reference's guard for a small sine; rs =
+// 1 / sin(theta).  The mixed form takes the sine of its FP32 angle instead: an
+// angle over its sine is only as good as the two go together (against FP64
+// sums, 3.6e-7 of a torque's scale with it, 4.3e-7 with rs of the cosine that
+// the arc cosine took).
 template<int TY, typename A>
-__device__ __forceinline__ A f4Dsin(A t) {
+__device__ __forceinline__ A f4Dsin(A t, A rs) {
 	A val = 0, m = 1;
 	A tt0 = t - (A) F4_T0[TY];
 	if(tt0 < 0) {
@@ -110,12 +141,43 @@ __device__ __forceinline__ A f4Dsin(A t) {
 		m = -1;
 	}
 	if(tt0 < (A) F4_TC[TY]) {
-		const A sint = sin(t);
-		if(tt0 > (A) F4_TS[TY]) val = m * 2 * (A) F4_B[TY] * (tt0 - (A) F4_TC[TY]) / sint;
-		else if(SQR(sint) > A(1e-8)) val = -m * 2 * (A) F4_A[TY] * tt0 / sint;
-		else val = -m * 2 * (A) F4_A[TY];
+		if constexpr(std::is_same<A, double>::value) {
+			if(tt0 > (A) F4_TS[TY]) val = m * 2 * (A) F4_B[TY] * (tt0 - (A) F4_TC[TY]) * rs;
+			else if(SQR(rs) < A(1e8)) val = -m * 2 * (A) F4_A[TY] * tt0 * rs;
+			else val = -m * 2 * (A) F4_A[TY];
+		}
+		else {
+			const A sint = sin_angle(t);
+			if(tt0 > (A) F4_TS[TY]) val = m * 2 * (A) F4_B[TY] * (tt0 - (A) F4_TC[TY]) / sint;
+			else if(SQR(sint) > A(1e-8)) val = -m * 2 * (A) F4_A[TY] * tt0 / sint;
+			else val = -m * 2 * (A) F4_A[TY];
+		}
 	}
 	return val;
+}
+
+// Whether f4<TY> of the angle of cosine c can be other than zero: the
+// cosines of F4_T0 +- F4_TC, widened by 1e-4 (FP32 rounding is below 1e-6).
+// Most pairs in a term's radial range fail one of its windows, and what they
+// skip are four to six arc cosines; a wave runs a term whenever one of its
+// lanes needs it.  24,576 nt in 24 batched systems, a launch: mixed 47 -> 45 us,
+// with sin_angle for the library's sine 33 us; all-FP64 68 us, 49 with this
+// and rsin.
+constexpr double cos_series(double x) {
+	double sum = 1., term = 1.;
+	for(int k = 1; k <= 20; k++) {
+		term *= -x * x / ((2 * k - 1) * (2 * k));
+		sum += term;
+	}
+	return sum;
+}
+
+template<int TY>
+__device__ __forceinline__ bool f4_open(float c) {
+	constexpr double T0 = F4_T0[TY], TC = F4_TC[TY];
+	constexpr float LO = T0 + TC < (double) PIf ? (float) (cos_series(T0 + TC) - 1e-4) : -2.f;
+	constexpr float HI = T0 - TC > 0. ? (float) (cos_series(T0 - TC) + 1e-4) : 2.f;
+	return c > LO && c < HI;
 }
 
 template<int TY>
@@ -280,10 +342,10 @@ __device__ void bonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv3 &
 	e[2] = es;
 	if(es != 0.) {
 		const double ff1D = f1D<1>(S, rstackmod, q.type, p.type);
-		const double f4t5Dsin = f4Dsin<STCK_T5, A>(pt5);
-		const double f4t6Dsin = f4Dsin<STCK_T6, A>(t6);
-		const double f4tB1Dsin = f4Dsin<STCK_TB1, A>(tB1);
-		const double f4tB2Dsin = f4Dsin<STCK_TB2, A>(tB2);
+		const double f4t5Dsin = f4Dsin<STCK_T5, A>(pt5, rsin_pi<1, A>(cost5));
+		const double f4t6Dsin = f4Dsin<STCK_T6, A>(t6, rsin<A>(cost6));
+		const double f4tB1Dsin = f4Dsin<STCK_TB1, A>(tB1, rsin<A>(costB1));
+		const double f4tB2Dsin = f4Dsin<STCK_TB2, A>(tB2, rsin<A>(costB2));
 		const double f5phi1D = f5D<STCK_PHI1>(cosphi1);
 		const double f5phi2D = f5D<STCK_PHI2>(cosphi2);
 
@@ -341,8 +403,21 @@ __device__ void nonbonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv
 
 	const dv3 &a1 = p.a1, &a3 = p.a3, &b1 = q.a1, &b3 = q.a3;
 	const double rbmod2 = dot(rbb, rbb);
+	// the windows of HB and CRST share their cosines
+	const bool hb_range = q.btype + p.btype == 3 && SQR((double) HYDR_RCLOW) < rbmod2 && rbmod2 < SQR((double) HYDR_RCHIGH);
+	const bool cr_range = SQR((double) F2_RCLOW[0]) < rbmod2 && rbmod2 < SQR((double) F2_RCHIGH[0]);
+	bool hb_open = false, cr_open = false;
+	if(hb_range || cr_range) {
+		const float inv = __builtin_amdgcn_rsqf((float) rbmod2);
+		const float c1 = -(float) dot(a1, b1), c4 = (float) dot(a3, b3), c2 = -(float) dot(b1, rbb) * inv, c3 = (float) dot(a1, rbb) * inv;
+		const float c7 = -(float) dot(b3, rbb) * inv, c8 = (float) dot(a3, rbb) * inv;
+		hb_open = hb_range && f4_open<HYDR_T1>(c1) && f4_open<HYDR_T2>(c2) && f4_open<HYDR_T3>(c3) && f4_open<HYDR_T4>(c4) &&
+				f4_open<HYDR_T7>(c7) && f4_open<HYDR_T8>(c8);
+		cr_open = cr_range && f4_open<CRST_T1>(c1) && f4_open<CRST_T2>(c2) && f4_open<CRST_T3>(c3) &&
+				(f4_open<CRST_T7>(c7) || f4_open<CRST_T7>(-c7)) && (f4_open<CRST_T8>(c8) || f4_open<CRST_T8>(-c8));
+	}
 	// hydrogen bonding (Watson-Crick-like pairs: base types summing to 3)
-	if(q.btype + p.btype == 3 && SQR((double) HYDR_RCLOW) < rbmod2 && rbmod2 < SQR((double) HYDR_RCHIGH)) {
+	if(hb_open) {
 		const double rhmod = sqrt(rbmod2);
 		if((double) HYDR_RCLOW < rhmod && rhmod < (double) HYDR_RCHIGH) {
 			const dv3 rhdir = rbb * (1. / rhmod);
@@ -359,12 +434,12 @@ __device__ void nonbonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv
 				const double ff1D = f1D<0>(S, rhmod, q.type, p.type);
 				// d f4(acos c) / dc = -f4Dsin, with the signs the reference's
 				// mesh derivatives carry
-				const double f4t1Dsin = -f4Dsin<HYDR_T1, A>(t1);
-				const double f4t2Dsin = -f4Dsin<HYDR_T2, A>(t2);
-				const double f4t3Dsin = f4Dsin<HYDR_T3, A>(t3);
-				const double f4t4Dsin = f4Dsin<HYDR_T4, A>(t4);
-				const double f4t7Dsin = -f4Dsin<HYDR_T7, A>(t7);
-				const double f4t8Dsin = f4Dsin<HYDR_T8, A>(t8);
+				const double f4t1Dsin = -f4Dsin<HYDR_T1, A>(t1, rsin<A>(cost1));
+				const double f4t2Dsin = -f4Dsin<HYDR_T2, A>(t2, rsin<A>(cost2));
+				const double f4t3Dsin = f4Dsin<HYDR_T3, A>(t3, rsin<A>(cost3));
+				const double f4t4Dsin = f4Dsin<HYDR_T4, A>(t4, rsin<A>(cost4));
+				const double f4t7Dsin = -f4Dsin<HYDR_T7, A>(t7, rsin<A>(cost7));
+				const double f4t8Dsin = f4Dsin<HYDR_T8, A>(t8, rsin<A>(cost8));
 				dv3 force = rhdir * (-ff1D * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8);
 				dv3 tl = cross(a3, b3) * (-(-ff1 * f4t1 * f4t2 * f4t3 * f4t4Dsin * f4t7 * f4t8));
 				tl -= cross(a1, b1) * (-ff1 * f4t1Dsin * f4t2 * f4t3 * f4t4 * f4t7 * f4t8);
@@ -382,12 +457,13 @@ __device__ void nonbonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv
 	}
 
 	// cross stacking, on the base-base separation
-	if(SQR((double) F2_RCLOW[0]) < rbmod2 && rbmod2 < SQR((double) F2_RCHIGH[0])) {
+	if(cr_open) {
 		const double rcmod = sqrt(rbmod2);
 		if((double) F2_RCLOW[0] < rcmod && rcmod < (double) F2_RCHIGH[0]) {
 			const dv3 rcdir = rbb * (1. / rcmod);
 			const double cost2 = -dot(b1, rcdir), cost3 = dot(a1, rcdir), cost7 = -dot(b3, rcdir), cost8 = dot(a3, rcdir);
-			const A t1 = lracos<A>(-dot(a1, b1)), t2 = lracos<A>(cost2), t3 = lracos<A>(cost3);
+			const double cost1 = -dot(a1, b1);
+			const A t1 = lracos<A>(cost1), t2 = lracos<A>(cost2), t3 = lracos<A>(cost3);
 			const A t7 = lracos<A>(cost7), t8 = lracos<A>(cost8);
 			const double ff2 = f2<0>(rcmod);
 			const double f4t1 = f4<CRST_T1, A>(t1), f4t2 = f4<CRST_T2, A>(t2), f4t3 = f4<CRST_T3, A>(t3);
@@ -397,11 +473,11 @@ __device__ void nonbonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv
 			e[2] = ec;
 			if(ec != 0.) {
 				const double ff2D = f2D<0>(rcmod);
-				const double f4t1Dsin = -f4Dsin<CRST_T1, A>(t1);
-				const double f4t2Dsin = -f4Dsin<CRST_T2, A>(t2);
-				const double f4t3Dsin = f4Dsin<CRST_T3, A>(t3);
-				const double f4t7Dsin = -f4Dsin<CRST_T7, A>(t7) + f4Dsin<CRST_T7, A>((A) PIf - t7);
-				const double f4t8Dsin = f4Dsin<CRST_T8, A>(t8) - f4Dsin<CRST_T8, A>((A) PIf - t8);
+				const double f4t1Dsin = -f4Dsin<CRST_T1, A>(t1, rsin<A>(cost1));
+				const double f4t2Dsin = -f4Dsin<CRST_T2, A>(t2, rsin<A>(cost2));
+				const double f4t3Dsin = f4Dsin<CRST_T3, A>(t3, rsin<A>(cost3));
+				const double f4t7Dsin = -f4Dsin<CRST_T7, A>(t7, rsin<A>(cost7)) + f4Dsin<CRST_T7, A>((A) PIf - t7, rsin_pi<1, A>(cost7));
+				const double f4t8Dsin = f4Dsin<CRST_T8, A>(t8, rsin<A>(cost8)) - f4Dsin<CRST_T8, A>((A) PIf - t8, rsin_pi<1, A>(cost8));
 				// the reference's theta4 factor is 1 here, its derivative 0
 				dv3 force = rcdir * (-(ff2D * f4t1 * f4t2 * f4t3 * f4t7 * f4t8));
 				dv3 tl = cross(a1, b1) * (-(-ff2 * f4t1Dsin * f4t2 * f4t3 * f4t7 * f4t8));
@@ -422,12 +498,20 @@ __device__ void nonbonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv
 	const dv3 pst = s_stack(p), qst = s_stack(q);
 	const dv3 rstack = sep(r, qst, pst);
 	const double rs2 = dot(rstack, rstack);
-	if(SQR((double) F2_RCLOW[1]) < rs2 && rs2 < SQR((double) F2_RCHIGH[1])) {
+	bool cx_open = SQR((double) F2_RCLOW[1]) < rs2 && rs2 < SQR((double) F2_RCHIGH[1]);
+	if(cx_open) {
+		// f4(t1) + f4(2 pi - t1): the second's window lies within the first's
+		const float inv = __builtin_amdgcn_rsqf((float) rs2), c5 = (float) dot(a3, rstack) * inv, c6 = (float) dot(b3, rstack) * inv;
+		cx_open = f4_open<CXST_T4>((float) dot(a3, b3)) && (f4_open<CXST_T5>(c5) || f4_open<CXST_T5>(-c5)) &&
+				(f4_open<CXST_T6>(c6) || f4_open<CXST_T6>(-c6)) && f4_open<CXST_T1>(-(float) dot(a1, b1));
+	}
+	if(cx_open) {
 		const double rsmod = sqrt(rs2);
 		if((double) F2_RCLOW[1] < rsmod && rsmod < (double) F2_RCHIGH[1]) {
 			const dv3 rsdir = rstack * (1. / rsmod);
 			const double cost5 = dot(a3, rsdir), cost6 = -dot(b3, rsdir);
-			const A t1 = lracos<A>(-dot(a1, b1)), t4 = lracos<A>(dot(a3, b3)), t5 = lracos<A>(cost5), t6 = lracos<A>(cost6);
+			const double cost1 = -dot(a1, b1), cost4 = dot(a3, b3);
+			const A t1 = lracos<A>(cost1), t4 = lracos<A>(cost4), t5 = lracos<A>(cost5), t6 = lracos<A>(cost6);
 			const double rbmod = sqrt(dot(rback, rback));
 			const dv3 rbdir = rback * (1. / rbmod);
 			const double cosphi3 = dot(rsdir, cross(rbdir, a1));
@@ -444,10 +528,10 @@ __device__ void nonbonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv
 			e[3] = ecx;
 			if(ecx != 0.) {
 				const double ff2D = f2D<1>(rsmod);
-				const double f4t1Dsin = -f4Dsin<CXST_T1, A>(t1) + f4Dsin<CXST_T1, A>(t1b);
-				const double f4t4Dsin = f4Dsin<CXST_T4, A>(t4);
-				const double f4t5Dsin = f4Dsin<CXST_T5, A>(t5) - f4Dsin<CXST_T5, A>((A) PIf - t5);
-				const double f4t6Dsin = -f4Dsin<CXST_T6, A>(t6) + f4Dsin<CXST_T6, A>((A) PIf - t6);
+				const double f4t1Dsin = -f4Dsin<CXST_T1, A>(t1, rsin<A>(cost1)) + f4Dsin<CXST_T1, A>(t1b, -rsin_pi<2, A>(cost1));
+				const double f4t4Dsin = f4Dsin<CXST_T4, A>(t4, rsin<A>(cost4));
+				const double f4t5Dsin = f4Dsin<CXST_T5, A>(t5, rsin<A>(cost5)) - f4Dsin<CXST_T5, A>((A) PIf - t5, rsin_pi<1, A>(cost5));
+				const double f4t6Dsin = -f4Dsin<CXST_T6, A>(t6, rsin<A>(cost6)) + f4Dsin<CXST_T6, A>((A) PIf - t6, rsin_pi<1, A>(cost6));
 				const double f5Dc3 = f5D<CXST_PHI3>(cosphi3);
 				const double f5Dc4 = f5D<CXST_PHI4>(cosphi4);
 				dv3 force = rsdir * (-ff2D * f4t1 * f4t4 * f4t5 * f4t6 * f5c3 * f5c4);
