@@ -60,8 +60,9 @@ struct oxh_batch {
 	std::vector<long long> target, done_steps;
 	double4 *bk_rlist = nullptr;
 	float4 *bk_blist = nullptr;
-	// page-locked word that a kernel writes for the host: the rebuild flag
-	// of a force call on the caller's buffers
+	// page-locked word that a kernel writes for the host (after the staging):
+	// the rebuild flag of a force call on the caller's buffers, or whether a
+	// chunk of steps left an error bit
 	int *h_flag = nullptr;
 	// what the host reads: page-locked staging (two halves), and the device
 	// buffer of what does not fit in STAGE_DIRECT
@@ -959,7 +960,9 @@ oxh_status alloc_stage(oxh_batch *B) {
 	size_t most = 0;
 	for(int s = 0; s < B->b.nsys; s++) most = std::max(most, (size_t) (B->pool ? B->cap[s] : B->n[s]) * 15 * sizeof(double));
 	B->stage_bytes = std::min(STAGE_MAX, std::max(std::max(most, (size_t) B->b.nsys * oxh::RED_W * sizeof(double)), (size_t) 4096));
-	if(hipHostMalloc((void **) &B->stage, B->stage_bytes, hipHostMallocPortable) != hipSuccess) return fail(OXH_ERR_ALLOC, "page-locked allocation failed");
+	// one block: the staging, then the word (each such allocation takes 60 us)
+	if(hipHostMalloc((void **) &B->stage, B->stage_bytes + sizeof(int), hipHostMallocPortable) != hipSuccess) return fail(OXH_ERR_ALLOC, "page-locked allocation failed");
+	B->h_flag = (int *) (B->stage + B->stage_bytes);
 	if(most <= STAGE_DIRECT) return OXH_OK;
 	for(hipEvent_t &e : B->stage_done) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 	return dalloc(B, &B->d_export, most / sizeof(double));
@@ -1426,7 +1429,6 @@ oxh_status oxh_batch_destroy(oxh_batch *B) {
 			b.raw_alt, b.step_need};
 	for(void *p : ptrs)
 		if(p) (void) hipFree(p);
-	if(B->h_flag) (void) hipHostFree(B->h_flag);
 	if(B->stage) (void) hipHostFree(B->stage);
 	if(B->d_export) (void) hipFree(B->d_export);
 	for(hipEvent_t e : B->stage_done)
@@ -1733,7 +1735,6 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 		if(any && !up(b.d_sys, b.h_sys.data(), n_sys * sizeof(oxh_sys))) return bail(fail(OXH_ERR_HIP, "system upload failed"));
 	}
 	TRYB(dalloc(B, &B->bk_rlist, N));
-	if(hipHostMalloc((void **) &B->h_flag, sizeof(int), hipHostMallocPortable) != hipSuccess) return bail(fail(OXH_ERR_ALLOC, "page-locked allocation failed"));
 	if(oxh_status r = alloc_stage(B); r != OXH_OK) return bail(r);
 	TRYB(dalloc(B, &b.any_rebuild, 1));
 	if(hipMemsetAsync(b.any_rebuild, 0, sizeof(int), st) != hipSuccess) return bail(fail(OXH_ERR_HIP, "memset failed"));
