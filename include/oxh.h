@@ -478,11 +478,11 @@ oxh_status oxh_batch_set_state(oxh_batch *b, int sys, const double *pos, const d
  * list; OXH_FAR_BACK=0 keeps every far pair within r_verlet, as the
  * reference's list does).
  * Shapes are picked by timing at upload (the all-FP64 mode times the lanes
- * only, in blocks of 64 with the far pairs inline; pools keep 8 lanes);
+ * and its far kernel, in blocks of 64; pools keep 8 lanes, packed);
  * OXH_FORCE_LANES / OXH_FAR_LANES fix them, OXH_PERSIST=0 disables the
  * workgroup engine, OXH_EDGE=0 / 1 forbids / forces the half-list form,
  * OXH_PACK=0 / 1 forbids / forces the packed form (never used with one
- * lane per nucleotide). */
+ * lane per nucleotide), OXH_FUSE=0 keeps one kernel per phase of a step. */
 oxh_status oxh_batch_stats(oxh_batch *b, double *out12);
 
 /* Average duration in ms of n back-to-back launches of the force kernel on
