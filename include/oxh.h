@@ -485,6 +485,13 @@ oxh_status oxh_batch_set_state(oxh_batch *b, int sys, const double *pos, const d
  * lane per nucleotide), OXH_FUSE=0 keeps one kernel per phase of a step. */
 oxh_status oxh_batch_stats(oxh_batch *b, double *out12);
 
+/* Which kernels the batch's work takes as it stands: out[0] 1 when
+ * oxh_batch_run takes one launch per MD step (state, lists, forces and
+ * integration in one kernel: grid-engine batches and pools of the mixed
+ * oxDNA2 form with the far pairs inline, lists built per particle and no
+ * external forces), else 0. */
+oxh_status oxh_batch_routes(oxh_batch *b, int *out1);
+
 /* Average duration in ms of n back-to-back launches of the force kernel on
  * the batch's stream, timed with HIP events (the reference times its steps
  * with CPU clocks around device syncs, src/Utilities/Timings.cpp:45-62). */

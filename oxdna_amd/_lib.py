@@ -23,7 +23,7 @@ EXPORTS = [
     "oxh_batch_destroy", "oxh_batch_update_lists", "oxh_batch_compute_forces", "oxh_batch_run",
     "oxh_batch_hilbert_sort", "oxh_batch_set_sort_interval", "oxh_batch_sync", "oxh_batch_get_state", "oxh_batch_get_forces", "oxh_batch_energies",
     "oxh_batch_energy_split", "oxh_batch_hb_count", "oxh_batch_get_pairs", "oxh_batch_system_info",
-    "oxh_batch_set_state", "oxh_batch_stats", "oxh_batch_time_forces", "oxh_hilbert_keys", "oxh_philox",
+    "oxh_batch_set_state", "oxh_batch_stats", "oxh_batch_routes", "oxh_batch_time_forces", "oxh_hilbert_keys", "oxh_philox",
     "oxh_pool_create", "oxh_pool_admit", "oxh_pool_release", "oxh_pool_status", "oxh_copy_bench", "oxh_batch_stress",
     "oxh_batch_fix_diffusion", "oxh_batch_set_fix_diffusion", "oxh_batch_checkpoint_bytes", "oxh_batch_save",
     "oxh_batch_restore", "oxh_batch_get_order", "oxh_batch_set_external_forces", "oxh_batch_get_images",
@@ -116,6 +116,7 @@ def lib():
         L.oxh_batch_system_info.argtypes = [V, I, P, P]
         L.oxh_batch_set_state.argtypes = [V, I, P, P, P, P, P]
         L.oxh_batch_stats.argtypes = [V, P]
+        L.oxh_batch_routes.argtypes = [V, P]
         L.oxh_batch_time_forces.argtypes = [V, I, P]
         L.oxh_hilbert_keys.argtypes = [I, I, P, P]
         L.oxh_philox.argtypes = [I, I, P, P, P]

@@ -370,6 +370,13 @@ class HIPBatch:
                     engine={0: "grid", 1: "workgroup", 2: "grid-edge"}[int(out[8])], n_systems=int(out[9]),
                     pack=bool(out[10]), far_back=int(out[11]))
 
+    def routes(self) -> dict:
+        """Which kernels the batch's work takes as it stands
+        (oxh_batch_routes)."""
+        out = np.zeros(1, np.int32)
+        check(lib().oxh_batch_routes(self.h, ptr(out)), "oxh_batch_routes")
+        return dict(one_launch=bool(out[0]))
+
 
 class HIPPool(HIPBatch):
     """A slot pool (oxh_pool_*): slots of fixed capacity that jobs are

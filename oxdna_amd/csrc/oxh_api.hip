@@ -2894,6 +2894,12 @@ oxh_status oxh_batch_stats(oxh_batch *B, double *out6) {  // 12 doubles
 	return OXH_OK;
 }
 
+oxh_status oxh_batch_routes(oxh_batch *B, int *out1) {
+	if(!B || !out1) return fail(OXH_ERR_ARG, "bad arguments");
+	out1[0] = !B->persist && fused_ok(B);
+	return OXH_OK;
+}
+
 }  // extern "C"
 
 // ---------------------------------------------------------------- checkpoints

@@ -1,0 +1,86 @@
+"""Which kernels a batch's steps take, and that the choice leaves no trace.
+
+`routes()` says whether steps take one launch each; the comparisons of
+test_gpu_fused.py are between two paths only if it differs between them, here
+for the same systems.  A trajectory has the same bits whichever path its steps
+take, whether the close pairs are evaluated packed or in place, and however a
+run is cut into calls (a chunk's first and last half steps are kernels of their
+own): bit for bit, since a pool's slots and a restored checkpoint rely on it.
+"""
+import numpy as np
+import pytest
+
+from test_gpu_fused import THERMO, _gas
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("pos", "a1", "a3", "vel", "L", "F", "T")
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from oxdna_amd import _lib, backend
+    assert _lib.device_count() >= 1, "no GPU visible"
+    return backend
+
+
+def _final(b, k):
+    F, T, _ = b.forces(k)
+    return dict(b.state(k), F=F, T=T)
+
+
+def _run(hip, monkeypatch, ss, steps, fuse=1, pack=0, lanes=8, **opts):
+    monkeypatch.setenv("OXH_FUSE", str(fuse))
+    monkeypatch.setenv("OXH_PACK", str(pack))
+    monkeypatch.setenv("OXH_PERSIST", "0")
+    monkeypatch.setenv("OXH_FORCE_LANES", str(lanes))
+    monkeypatch.setenv("OXH_FAR_LANES", "0")
+    per = [dict(seed=100 + k) for k in range(len(ss))]
+    with hip.HIPBatch(ss, options=per, dt=0.003, verlet_skin=0.05, refresh_vel=True, **opts) as b:
+        assert b.routes()["one_launch"] == bool(fuse)
+        for n in steps:
+            b.run(n)
+        assert b.routes()["one_launch"] == bool(fuse)
+        return [_final(b, k) for k in range(len(ss))]
+
+
+def _equal(x, y):
+    for a, b in zip(x, y):
+        for key in KEYS:
+            assert np.array_equal(a[key], b[key]), (key, np.abs(a[key] - b[key]).max())
+
+
+@pytest.mark.parametrize("thermo", list(THERMO))
+@pytest.mark.parametrize("sizes", [[(1, 5)], [(31, 19)], [(1, 9), (33, 17), (4, 21)]])
+def test_same_bits_on_every_path(hip, monkeypatch, thermo, sizes):
+    ss = [_gas(5 + k, n, bp) for k, (n, bp) in enumerate(sizes)]
+    want = _run(hip, monkeypatch, ss, [130], **THERMO[thermo])
+    _equal(want, _run(hip, monkeypatch, ss, [37, 1, 20, 72], **THERMO[thermo]))
+    _equal(want, _run(hip, monkeypatch, ss, [130], pack=1, **THERMO[thermo]))
+    _equal(want, _run(hip, monkeypatch, ss, [130], fuse=0, **THERMO[thermo]))
+    _equal(want, _run(hip, monkeypatch, ss, [65, 65], fuse=0, pack=1, **THERMO[thermo]))
+
+
+@pytest.mark.parametrize("lanes", [2, 4, 16, 32])
+def test_same_bits_for_other_lanes(hip, monkeypatch, lanes):
+    ss = [_gas(5, 1, 9), _gas(6, 33, 17), _gas(7, 7, 13)]
+    want = _run(hip, monkeypatch, ss, [96], lanes=lanes, **THERMO["langevin"])
+    _equal(want, _run(hip, monkeypatch, ss, [31, 65], lanes=lanes, pack=1, **THERMO["langevin"]))
+    _equal(want, _run(hip, monkeypatch, ss, [96], lanes=lanes, fuse=0, **THERMO["langevin"]))
+
+
+def test_paths_that_are_not_one_launch(hip, monkeypatch):
+    s = _gas(3, 30, 20)
+    with hip.HIPBatch(s, backend_precision="double") as b:
+        assert not b.routes()["one_launch"]
+    with hip.HIPBatch(_gas(3, 1, 9)) as b:      # workgroup engine
+        assert not b.routes()["one_launch"]
+    monkeypatch.setenv("OXH_FORCE_LANES", "8")
+    monkeypatch.setenv("OXH_FAR_LANES", "8")
+    with hip.HIPBatch(s) as b:
+        assert not b.routes()["one_launch"]
+    monkeypatch.setenv("OXH_FAR_LANES", "0")
+    with hip.HIPBatch(s) as b:
+        assert b.routes()["one_launch"]
+        b.set_external_forces([dict(type="trap", particle=0, stiff=1.0, pos0=s.pos[0], dir=(0.0, 0.0, 1.0))])
+        assert not b.routes()["one_launch"]
