@@ -489,7 +489,8 @@ oxh_status oxh_batch_stats(oxh_batch *b, double *out12);
  * oxh_batch_run takes one launch per MD step (state, lists, forces and
  * integration in one kernel: grid-engine batches and pools of the mixed
  * oxDNA2 form with the far pairs inline, lists built per particle and no
- * external forces), else 0. */
+ * external forces; systems with rows above 512 entries have theirs built by a
+ * launch of their own before it), else 0. */
 oxh_status oxh_batch_routes(oxh_batch *b, int *out1);
 
 /* Average duration in ms of n back-to-back launches of the force kernel on

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -411,6 +412,8 @@ void enqueue_fused(oxh_batch *B, int count, long long step_index0) {
 	oxh::launch_step_begin(b.stream, 3 * nneed, b.step_need, 3 * ncell, b.cell_count);
 	oxh::StepArgs a = step_args(B);
 	bool alt = false;   // the current state is in the other buffers
+	bool any_long = false;
+	for(const oxh_sys &S : b.h_sys) any_long |= S.long_rows != 0;
 	auto buffers = [&](bool in_alt, bool out_alt, int k) {
 		a.pos = in_alt ? b.pos_alt : b.pos;
 		a.q64 = in_alt ? b.q64_alt : b.q64;
@@ -438,6 +441,7 @@ void enqueue_fused(oxh_batch *B, int count, long long step_index0) {
 	for(int k = 0; k < count; k++) {
 		const bool go_on = k + 1 < count && !bussi_due(k);
 		buffers(alt, go_on ? !alt : alt, k);
+		if(any_long) oxh::launch_step_long_rows(b.stream, a);
 		oxh::launch_step(b.stream, a, b.lanes, b.pack, b.force_block, k, go_on);
 		if(go_on) {
 			alt = !alt;
@@ -523,15 +527,17 @@ oxh_status alloc_cell_slots(oxh_batch *B, int cap) {
 	return OXH_OK;
 }
 
-// doubles the neighbour, cell or edge-row capacity after an overflow and
-// clears the overflow bits (the caller rebuilds)
+// doubles the neighbour, cell or edge-row capacity after an overflow (or
+// notes a system's long rows) and clears the overflow bits (the caller
+// rebuilds)
 oxh_status grow_lists(oxh_batch *B, const std::vector<oxh_sys_state> &st) {
 	oxh::Batch &b = B->b;
-	bool grow_neigh = false, grow_cells = false, grow_edge = false;
-	for(auto &s : st) {
+	bool grow_neigh = false, grow_cells = false, grow_edge = false, long_rows = false;
+	for(size_t k = 0; k < st.size(); k++) {
+		const oxh_sys_state &s = st[k];
+		if(s.error & oxh::ERR_ROW) b.h_sys[k].long_rows = long_rows = 1;
 		if(s.error & oxh::ERR_LIST) grow_neigh = true;
 		if(s.error & oxh::ERR_CELLS) grow_cells = true;
-		if(s.error & oxh::ERR_ROW) b.fuse = false;
 		// a row overflow empties the row, which its partners report as well
 		if((s.error & oxh::ERR_EDGE) && !(s.error & oxh::ERR_LIST)) grow_edge = true;
 	}
@@ -544,6 +550,7 @@ oxh_status grow_lists(oxh_batch *B, const std::vector<oxh_sys_state> &st) {
 	}
 	if(grow_cells && b.ncell_total) TRY(alloc_cell_slots(B, b.cell_cap * 2));
 	if(grow_edge && b.ecap > 0) TRY(alloc_edges(B, std::min(2 * b.ecap, b.max_neigh)));
+	if(long_rows) HIPCHK(hipMemcpyAsync(b.d_sys, b.h_sys.data(), b.nsys * sizeof(oxh_sys), hipMemcpyHostToDevice, b.stream));
 	k_clear_err<<<(b.nsys + 63) / 64, 64, 0, b.stream>>>(b.nsys, b.d_state, oxh::ERR_OVERFLOW);
 	if(b.graph_exec) {
 		(void) hipGraphExecDestroy(b.graph_exec);
@@ -1993,17 +2000,19 @@ oxh_status oxh_batch_run(oxh_batch *B, long long n_steps) {
 		// the systems' states only when one of them has something to say
 		std::vector<oxh_sys_state> st;
 		if(*(volatile int *) B->h_flag) TRY(read_states(B, st));
-		bool overflow = false;
+		bool overflow = false, grows = false;
 		int bad = -1, bad_ext = -1;
 		for(int s = 0; s < (int) st.size(); s++) {
 			if(st[s].error & oxh::ERR_OVERFLOW) overflow = true;
+			if(st[s].error & oxh::ERR_OVERFLOW & ~oxh::ERR_ROW) grows = true;
 			if((st[s].error & 1) && bad < 0) bad = s;
 			if((st[s].error & oxh::ERR_EXT) && bad_ext < 0) bad_ext = s;
 		}
 		if(overflow) {
 			// replay the chunk from its start with larger buffers and the
-			// same lists
-			if(++retries > 8) return fail(OXH_ERR_SYSTEM, "neighbour list keeps overflowing");
+			// same lists (a system's long rows are found once, so those
+			// replays are as many as systems at most)
+			if(grows && ++retries > 8) return fail(OXH_ERR_SYSTEM, "neighbour list keeps overflowing");
 			TRY(restore(B));
 			TRY(grow_lists(B, st));
 			TRY(rebuild_from_rlist(B));
@@ -2138,9 +2147,14 @@ oxh_status oxh_pool_release(oxh_batch *B, int slot) {
 	oxh::Batch &b = B->b;
 	HIPCHK(hipStreamSynchronize(b.stream));
 	oxh_sys &S = b.h_sys[slot];
+	if(S.long_rows && b.graph_exec) {   // its steps have a launch for them
+		(void) hipGraphExecDestroy(b.graph_exec);
+		b.graph_exec = nullptr;
+	}
 	S.n = 0;
 	S.use_cells = 0;
 	S.ncell = 0;
+	S.long_rows = 0;
 	B->n[slot] = 0;
 	B->target[slot] = B->done_steps[slot] = 0;
 	oxh_sys_state hst;
@@ -2925,7 +2939,7 @@ unsigned long long systems_fingerprint(const oxh_batch *B) {
 		S.has_ext = 0;        // external forces are set again after a restore
 		S.ext_step0 = 0;
 		const unsigned char *c = (const unsigned char *) &S;
-		for(size_t k = 0; k < sizeof(S); k++) {
+		for(size_t k = 0; k < offsetof(oxh_sys, long_rows); k++) {   // found again by the restored run
 			h ^= c[k];
 			h *= 1099511628211ull;
 		}

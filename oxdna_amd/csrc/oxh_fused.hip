@@ -19,7 +19,8 @@
 // an atomic per nucleotide next to ~20 us of forces.  Cells hold their
 // particles in arrival order; a row is put in the lists' order (cell, then
 // index) by ranking its entries, so rows and forces are those of the other
-// path.
+// path.  Rows above STEP_ROW entries have a launch of their own before the
+// step's, for the systems that have met one.
 // Measured, per MD step: 24,576-nt gas with Bussi 39 -> 35 us, 777 nt without
 // cells 20 -> 17 us, a pool of eight jobs of 259 to 1,332 nt 44 -> 41 us.
 // Not for dense batches (their lists are built cell by cell), far pairs in a
@@ -42,117 +43,85 @@ namespace {
 // pairs from the front, far pairs from the back
 constexpr int GROUP = BUILD_LANES;
 
+// what decides whether j enters the row of particle i of a system with
+// cells, as in build_row; the backbone sites are those of this state, which
+// the row records (blist)
+struct Candidates {
+	const oxh_sys &S;
+	const StepArgs &a;
+	int i;
+	double4 p;
+	int2 bd;
+	bool back;
+	float4 p32, bi;
+	__device__ __forceinline__ Candidates(int i_, const oxh_sys &S_, const StepArgs &a_) : S(S_), a(a_), i(i_) {
+		p = a.pos[i];
+		bd = a.bonds[i];
+		back = S.far_back != 0;
+		p32 = a.pos32[i];
+		bi = back ? a.bpos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+	}
+	__device__ __forceinline__ void test(int j, bool &close, bool &far) const {
+		close = far = false;
+		if(j < 0 || j == i || j == bd.x || j == bd.y) return;
+		const float db2 = back ? back_dist2(bi, a.bpos[j], S) : 0.f;
+		if(back && !(db2 < S.rgate2f)) return;
+		classify_pair(S, p, p32, a.pos32[j], a.pos, j, true, close, far);
+		if(far && back && !(db2 < S.rbf2)) far = false;
+	}
+};
+
 // Row of particle i of a system with cells whose particles lie in the cells'
 // arrival order (the 32 lanes of a group call it): the candidates, tests and
-// row order of build_row.  bsite: the backbone sites of this state, which
-// are the ones the row records (blist).
+// row order of build_row.
 __device__ __forceinline__ void build_row_binned(int i, int l, int s, const StepArgs &a, unsigned int *keys) {
 	constexpr int K = GROUP;
 	const oxh_sys &S = a.systems[s];
-	const double4 p = a.pos[i];
-	const int2 bd = a.bonds[i];
-	const bool back = S.far_back != 0;
-	const float4 p32 = a.pos32[i];
-	const float4 bi = back ? a.bpos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+	const Candidates cand(i, S, a);
 	const int g0 = (threadIdx.x & 63) & ~(K - 1);
 	const uint64_t gmask = ((1ull << K) - 1ull) << g0;
 	const uint64_t below = ((1ull << (threadIdx.x & 63)) - 1ull) & gmask;
+	int *row = a.nbr + (size_t) i * a.max_neigh;
+	const Stencil n = stencil_of(cand.p, cand.p32, S);
 	int nc = 0, nf = 0;
 	bool full = false;
-	const int cx = cell_coord(p.x, S.inv_box[0], S.nc[0]);
-	const int cy = cell_coord(p.y, S.inv_box[1], S.nc[1]);
-	const int cz = cell_coord(p.z, S.inv_box[2], S.nc[2]);
-	const int R = S.stencil, W = 2 * R + 1, NS = W * W * W;
-	const float ux = p32.x - cx * S.cell_w[0], uy = p32.y - cy * S.cell_w[1], uz = p32.z - cz * S.cell_w[2];
-	const float cull = (sqrtf(S.rv2f) + 1e-3f) * (sqrtf(S.rv2f) + 1e-3f);
-	auto gap = [](int o, float u, float w) { return o > 0 ? o * w - u : (o < 0 ? u + (-o - 1) * w : 0.f); };
-	auto stream = [&](auto rounds_tag) {
-		constexpr int ROUNDS = decltype(rounds_tag)::value;
-		int cell[ROUNDS], excl[ROUNDS], base[ROUNDS + 1];
-		base[0] = 0;
-#pragma unroll
-		for(int r = 0; r < ROUNDS; r++) {
-			const int k = l + K * r;
-			int cnt = 0;
-			cell[r] = 0;
-			if(k < NS) {
-				const int oz = k / (W * W) - R, oy = (k / W) % W - R, ox = k % W - R;
-				const float gx = gap(ox, ux, S.cell_w[0]), gy = gap(oy, uy, S.cell_w[1]), gz = gap(oz, uz, S.cell_w[2]);
-				if(gx * gx + gy * gy + gz * gz <= cull) {
-					int z = cz + oz, y = cy + oy, x = cx + ox;
-					z += (z < 0) ? S.nc[2] : (z >= S.nc[2] ? -S.nc[2] : 0);
-					y += (y < 0) ? S.nc[1] : (y >= S.nc[1] ? -S.nc[1] : 0);
-					x += (x < 0) ? S.nc[0] : (x >= S.nc[0] ? -S.nc[0] : 0);
-					cell[r] = S.cell_first + (z * S.nc[1] + y) * S.nc[0] + x;
-					const int held = a.count[cell[r]];
-					full |= held > a.cell_cap;
-					cnt = min(held, a.cell_cap);
+	walk_stencil(
+			n, l, S,
+			[&](int c) {
+				const int held = a.count[c];
+				full |= held > a.cell_cap;
+				return min(held, a.cell_cap);
+			},
+			[&](int c, int slot, int kc) {
+				const int j = slot >= 0 ? a.raw[(size_t) c * a.cell_cap + slot] : -1;
+				bool close, far;
+				cand.test(j, close, far);
+				const uint64_t bc = __ballot(close) & gmask, bf = __ballot(far) & gmask;
+				const unsigned int key = ((unsigned int) kc << 24) | (unsigned int) j;
+				if(close) {
+					const int q = nc + __popcll(bc & below);
+					if(q + nf < STEP_ROW) keys[q] = key;
 				}
-			}
-			int incl = cnt;
-			for(int off = 1; off < K; off <<= 1) {
-				const int v = __shfl_up(incl, off, K);
-				if(l >= off) incl += v;
-			}
-			excl[r] = incl - cnt;
-			base[r + 1] = base[r] + __shfl(incl, K - 1, K);
-		}
-		const int total = base[ROUNDS];
-		for(int m0 = 0; m0 < total; m0 += K) {
-			const int g = m0 + l;
-			int c = 0, slot = 0, kc = 0;
-#pragma unroll
-			for(int r = 0; r < ROUNDS; r++) {
-				const int gr = g - base[r];
-				int lo = 0;
-				for(int step = K >> 1; step > 0; step >>= 1)
-					if(__shfl(excl[r], lo + step, K) <= gr) lo += step;
-				const int cr = __shfl(cell[r], lo, K), sr = gr - __shfl(excl[r], lo, K);
-				if(g >= base[r] && g < base[r + 1]) {
-					c = cr;
-					slot = sr;
-					kc = lo + K * r;
+				if(far) {
+					const int q = nf + __popcll(bf & below);
+					if(nc + q < STEP_ROW) keys[STEP_ROW - 1 - q] = key;
 				}
-			}
-			const int j = g < total ? a.raw[(size_t) c * a.cell_cap + slot] : -1;
-			bool close = false, far = false;
-			if(j >= 0 && j != i && j != bd.x && j != bd.y) {
-				const float db2 = back ? back_dist2(bi, a.bpos[j], S) : 0.f;
-				if(!back || db2 < S.rgate2f) {
-					classify_pair(S, p, p32, a.pos32[j], a.pos, j, true, close, far);
-					if(far && back && !(db2 < S.rbf2)) far = false;
-				}
-			}
-			const uint64_t bc = __ballot(close) & gmask, bf = __ballot(far) & gmask;
-			const unsigned int key = ((unsigned int) kc << 24) | (unsigned int) j;
-			if(close) {
-				const int q = nc + __popcll(bc & below);
-				if(q + nf < STEP_ROW) keys[q] = key;
-			}
-			if(far) {
-				const int q = nf + __popcll(bf & below);
-				if(nc + q < STEP_ROW) keys[STEP_ROW - 1 - q] = key;
-			}
-			nc += __popcll(bc);
-			nf += __popcll(bf);
-		}
-	};
-	if(R == 1) stream(std::integral_constant<int, 1>());
-	else stream(std::integral_constant<int, 4>());
+				nc += __popcll(bc);
+				nf += __popcll(bf);
+			});
 	full = (__ballot(full) & gmask) != 0;
 	if(nc + nf > min(a.max_neigh, STEP_ROW) || full) {
 		if(l == 0) {
 			atomicOr(&a.state[s].error,
 					(full ? ERR_CELLS : 0) | (nc + nf > a.max_neigh ? ERR_LIST : 0) | (nc + nf > STEP_ROW ? ERR_ROW : 0));
 			a.nnbr[i] = make_int2(0, 0);
-			a.rlist[i] = p;
-			if(back) a.blist[i] = bi;
+			a.rlist[i] = cand.p;
+			if(cand.back) a.blist[i] = cand.bi;
 		}
 		return;
 	}
 	// the keys' ranks are the entries' places
 	__threadfence_block();
-	int *row = a.nbr + (size_t) i * a.max_neigh;
 	for(int e = l; e < nc; e += K) {
 		const unsigned int key = keys[e];
 		int rank = 0;
@@ -168,8 +137,8 @@ __device__ __forceinline__ void build_row_binned(int i, int l, int s, const Step
 	}
 	if(l != 0) return;
 	a.nnbr[i] = make_int2(nc, nf);
-	a.rlist[i] = p;
-	if(back) a.blist[i] = bi;
+	a.rlist[i] = cand.p;
+	if(cand.back) a.blist[i] = cand.bi;
 }
 
 // Rows of RB particles of a system without cells (row[r] < 0: none), the
@@ -227,6 +196,72 @@ __device__ __forceinline__ void build_rows_all(const int (&row)[RB], int l, int 
 		a.nnbr[row[r]] = over ? make_int2(0, 0) : make_int2(nc[r], nf[r]);
 		a.rlist[row[r]] = p[r];
 	}
+}
+
+// Rows of a system that has rows longer than the keys held, before the step's
+// own launch: cell after cell, an entry's place is the number of its cell's
+// entries before it, so a row of any length comes out in the same order.  In
+// k_step itself this code cost every other batch 0.9 % (24,576-nt gas), on
+// scalar registers; so the step's kernel is the same for all systems of a
+// pool, whatever their rows, and only this launch comes on top.
+__global__ void __launch_bounds__(256) k_step_long_rows(StepArgs a) {
+	constexpr int K = GROUP;
+	if(!a.need[a.nsys]) return;
+	const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t / K, l = t % K;
+	if(i >= a.N) return;
+	const int s = a.pinfo[i].y;
+	const oxh_sys &S = a.systems[s];
+	if(!S.long_rows || !a.need[s] || padding(i, S)) return;
+	const Candidates cand(i, S, a);
+	const int g0 = (threadIdx.x & 63) & ~(K - 1);
+	const uint64_t gmask = ((1ull << K) - 1ull) << g0;
+	int *row = a.nbr + (size_t) i * a.max_neigh;
+	const Stencil n = stencil_of(cand.p, cand.p32, S);
+	int nc = 0, nf = 0;
+	bool full = false;
+	for(int oz = -n.R; oz <= n.R; oz++)
+		for(int oy = -n.R; oy <= n.R; oy++)
+			for(int ox = -n.R; ox <= n.R; ox++) {
+				bool in_range;
+				const int c = stencil_cell(n, oz, oy, ox, S, in_range);
+				const int all = in_range ? a.count[c] : 0, held = min(all, a.cell_cap);
+				full |= all > a.cell_cap;
+				const int *in = a.raw + (size_t) c * a.cell_cap;
+				int cc = 0, cf = 0;
+				for(int m0 = 0; m0 < held; m0 += K) {
+					const int j = m0 + l < held ? in[m0 + l] : -1;
+					bool close = false, far = false;
+					int rc = 0, rf = 0;
+					for(int o0 = 0; o0 < held; o0 += K) {
+						const int jo = o0 + l < held ? in[o0 + l] : -1;
+						bool oc, of;
+						cand.test(jo, oc, of);
+						if(o0 == m0) {
+							close = oc;
+							far = of;
+						}
+						uint64_t bc = __ballot(oc) >> g0, bf = __ballot(of) >> g0;
+#pragma unroll 1
+						for(int t = 0; t < K; t++, bc >>= 1, bf >>= 1) {
+							const bool before = __shfl(jo, t, K) < j;
+							rc += before && (bc & 1);
+							rf += before && (bf & 1);
+						}
+					}
+					if(close && nc + rc < a.max_neigh) row[nc + rc] = j;
+					if(far && nf + rf < a.max_neigh) row[a.max_neigh - 1 - nf - rf] = j;
+					cc += __popcll(__ballot(close) & gmask);
+					cf += __popcll(__ballot(far) & gmask);
+				}
+				nc += cc;
+				nf += cf;
+			}
+	if(l != 0) return;
+	const bool over = nc + nf > a.max_neigh || full;
+	if(over) atomicOr(&a.state[s].error, (full ? ERR_CELLS : 0) | (nc + nf > a.max_neigh ? ERR_LIST : 0));
+	a.nnbr[i] = over ? make_int2(0, 0) : make_int2(nc, nf);
+	a.rlist[i] = cand.p;
+	if(cand.back) a.blist[i] = cand.bi;
 }
 
 // particle i of step k: into its cell (slot in arrival order) and its
@@ -340,7 +375,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 				const int si = a.pinfo[i].y;
 				const oxh_sys &S = a.systems[si];
 				if(!a.need[si] || padding(i, S)) continue;
-				if(S.use_cells) build_row_binned(i, l, si, a, sh.keys[grp]);
+				if(S.use_cells) {
+					if(!S.long_rows) build_row_binned(i, l, si, a, sh.keys[grp]);
+				}
 				else {
 					const int alone[1] = {i};
 					build_rows_all<1>(alone, l, si, a);
@@ -391,6 +428,11 @@ void launch_step_begin(hipStream_t st, int nneed, int *need, int ncount, int *co
 }
 
 void launch_step_first(hipStream_t st, const StepArgs &a, int k) { k_step_first<<<(a.N + 255) / 256, 256, 0, st>>>(a, k); }
+
+void launch_step_long_rows(hipStream_t st, const StepArgs &a) {
+	const size_t threads = (size_t) a.N * GROUP;
+	k_step_long_rows<<<(unsigned) ((threads + 255) / 256), 256, 0, st>>>(a);
+}
 
 void launch_step(hipStream_t st, const StepArgs &a, int lanes, bool pack, int block, int k, bool go_on) {
 	switch(lanes) {

@@ -148,7 +148,7 @@ struct Batch {
 // oxh_sys_state.error bits
 constexpr int ERR_BOND = 1, ERR_LIST = 2, ERR_CELLS = 4, ERR_EDGE = 8;
 constexpr int ERR_EXT = 16;   // a particle where an external force is undefined (the reference throws)
-constexpr int ERR_ROW = 32;   // a row longer than k_step sorts in LDS: the batch goes on with one kernel per phase
+constexpr int ERR_ROW = 32;   // a row longer than k_step sorts in LDS: k_step_long_rows builds this system's from then on
 constexpr int ERR_OVERFLOW = ERR_LIST | ERR_CELLS | ERR_EDGE | ERR_ROW;   // fixed by growing a buffer and replaying
 
 constexpr int RED_CHUNK = 2048;
@@ -216,12 +216,14 @@ struct StepArgs {
 	int *raw, *raw_next;
 	float4 *pos32, *pos32_next;
 };
-// longest list row of a system with cells, and largest batch, that k_step
-// builds (a row's keys wait in LDS, (stencil cell << 24) | particle)
+// longest list row of a system with cells that k_step itself builds (a system
+// with a longer one has long_rows set), and largest batch (a row's keys wait
+// in LDS, (stencil cell << 24) | particle)
 constexpr int STEP_ROW = 512, STEP_MAX_N = 1 << 24;
 bool fused_lanes(int lanes);
 void launch_step_begin(hipStream_t st, int nneed, int *need, int ncount, int *count);
 void launch_step_first(hipStream_t st, const StepArgs &a, int k);
+void launch_step_long_rows(hipStream_t st, const StepArgs &a);
 void launch_step(hipStream_t st, const StepArgs &a, int lanes, bool pack, int block, int k, bool go_on);
 void launch_reduce(hipStream_t st, const Batch &b, double *out = nullptr);   // out: elsewhere than red_out
 // velocities ~ N(0, T) for particles [i0, i0 + n)

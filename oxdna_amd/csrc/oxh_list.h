@@ -78,6 +78,108 @@ __device__ __forceinline__ void classify_pair(const oxh_sys &S, double4 p, float
 	}
 }
 
+// The cells within +-R of a particle's cell (27 or 125; cell k = (oz + R) W^2
+// + (oy + R) W + ox + R), and the particle's place inside its cell, for the
+// distance to the others.
+struct Stencil {
+	int cx, cy, cz, R, W, NS;
+	float ux, uy, uz, cull;
+};
+
+__device__ __forceinline__ Stencil stencil_of(double4 p, float4 p32, const oxh_sys &S) {
+	Stencil n;
+	n.cx = cell_coord(p.x, S.inv_box[0], S.nc[0]);
+	n.cy = cell_coord(p.y, S.inv_box[1], S.nc[1]);
+	n.cz = cell_coord(p.z, S.inv_box[2], S.nc[2]);
+	n.R = S.stencil;
+	n.W = 2 * n.R + 1;
+	n.NS = n.W * n.W * n.W;
+	n.ux = p32.x - n.cx * S.cell_w[0];
+	n.uy = p32.y - n.cy * S.cell_w[1];
+	n.uz = p32.z - n.cz * S.cell_w[2];
+	// a cell is culled when its nearest point is farther than r_verlet by a
+	// margin far above the FP32 error of these distances
+	n.cull = (sqrtf(S.rv2f) + 1e-3f) * (sqrtf(S.rv2f) + 1e-3f);
+	return n;
+}
+
+// the batch's index of the cell at offsets oz, oy, ox, and whether any of it
+// is in range
+__device__ __forceinline__ int stencil_cell(const Stencil &n, int oz, int oy, int ox, const oxh_sys &S, bool &in_range) {
+	auto gap = [](int o, float u, float w) { return o > 0 ? o * w - u : (o < 0 ? u + (-o - 1) * w : 0.f); };
+	const float gx = gap(ox, n.ux, S.cell_w[0]), gy = gap(oy, n.uy, S.cell_w[1]), gz = gap(oz, n.uz, S.cell_w[2]);
+	in_range = gx * gx + gy * gy + gz * gz <= n.cull;
+	int z = n.cz + oz, y = n.cy + oy, x = n.cx + ox;
+	z += (z < 0) ? S.nc[2] : (z >= S.nc[2] ? -S.nc[2] : 0);
+	y += (y < 0) ? S.nc[1] : (y >= S.nc[1] ? -S.nc[1] : 0);
+	x += (x < 0) ? S.nc[0] : (x >= S.nc[0] ? -S.nc[0] : 0);
+	return S.cell_first + (z * S.nc[1] + y) * S.nc[0] + x;
+}
+
+// the same for cell k
+__device__ __forceinline__ int stencil_cell(const Stencil &n, int k, const oxh_sys &S, bool &in_range) {
+	return stencil_cell(n, k / (n.W * n.W) - n.R, (k / n.W) % n.W - n.R, k % n.W - n.R, S, in_range);
+}
+
+// The candidates of a particle of a system with cells, in chunks of one per
+// lane (the 32 lanes of a group call it): test(cell, slot, k) with the
+// candidates in the order of the stencil's cells k, then of their slots
+// (slot < 0: none for this lane).  held(cell) is a cell's occupancy.  Lane l
+// takes cells l, l + 32, ... (1 round for 27 cells, 4 for 125); lane prefix
+// sums of the occupancies number the candidates, and each lane finds its
+// candidate's cell by a binary search over them: the cells' loads overlap
+// instead of following each other.
+template<class Held, class Test>
+__device__ __forceinline__ void walk_stencil(const Stencil &n, int l, const oxh_sys &S, Held &&held, Test &&test) {
+	constexpr int K = BUILD_LANES;
+	// the stencil is a compile-time constant of each branch
+	auto stream = [&](auto rounds_tag) {
+		constexpr int ROUNDS = decltype(rounds_tag)::value;
+		int cell[ROUNDS], excl[ROUNDS], base[ROUNDS + 1];
+		base[0] = 0;
+#pragma unroll
+		for(int r = 0; r < ROUNDS; r++) {
+			const int k = l + K * r;
+			int cnt = 0;
+			cell[r] = 0;
+			if(k < n.NS) {
+				bool in_range;
+				cell[r] = stencil_cell(n, k, S, in_range);
+				if(in_range) cnt = held(cell[r]);
+			}
+			int incl = cnt;
+			for(int off = 1; off < K; off <<= 1) {
+				const int v = __shfl_up(incl, off, K);
+				if(l >= off) incl += v;
+			}
+			excl[r] = incl - cnt;
+			base[r + 1] = base[r] + __shfl(incl, K - 1, K);
+		}
+		const int total = base[ROUNDS];
+		for(int m0 = 0; m0 < total; m0 += K) {
+			const int g = m0 + l;
+			int c = 0, slot = -1, kc = 0;
+#pragma unroll
+			for(int r = 0; r < ROUNDS; r++) {
+				// candidates base[r] .. base[r + 1] - 1 come from round r
+				const int gr = g - base[r];
+				int lo = 0;
+				for(int step = K >> 1; step > 0; step >>= 1)
+					if(__shfl(excl[r], lo + step, K) <= gr) lo += step;
+				const int cr = __shfl(cell[r], lo, K), sr = gr - __shfl(excl[r], lo, K);
+				if(g >= base[r] && g < base[r + 1]) {
+					c = cr;
+					slot = sr;
+					kc = lo + K * r;
+				}
+			}
+			test(c, slot, kc);
+		}
+	};
+	if(n.R == 1) stream(std::integral_constant<int, 1>());
+	else stream(std::integral_constant<int, 4>());
+}
+
 // BUILD_LANES threads per particle share the candidate scan: in every chunk
 // each lane tests one candidate, a wave ballot gives every passing lane its
 // slot, so the row is written in candidate order whatever the timing.
@@ -85,15 +187,8 @@ __device__ __forceinline__ void classify_pair(const oxh_sys &S, double4 p, float
 // the back.  A pair cannot come closer than R_CLOSE before the next rebuild
 // unless it is within R_CLOSE + 2 skin now, so far pairs only ever need
 // Debye-Hueckel.
-// With cells, the candidates are the particles of the cells within
-// +-stencil of the particle's cell (27 or 125 cells; k = (oz + R) W^2 +
-// (oy + R) W + ox + R), minus the cells whose nearest point is out of
-// range.  With K = 32 lanes, lane l takes cells l, l + 32, ...; lane prefix
-// sums of the cells' occupancies number the candidates (cells in k order,
-// each cell's items sorted by particle index), and the group scans them in
-// chunks of K, each lane finding its candidate's cell by a binary search
-// over the prefix sums: the cells' loads overlap instead of following each
-// other.
+// With cells, the candidates are the particles of the stencil's cells
+// (walk_stencil), each cell's items sorted by particle index.
 // Every lane of the group must call it; lane 0 writes the row's counts and
 // the list position.
 template<int K>
@@ -136,80 +231,16 @@ __device__ __forceinline__ void build_row(int i, int l, int s, const double4 *__
 		nf += __popcll(bf);
 	};
 	if(S.use_cells) {
-		const int cx = cell_coord(p.x, S.inv_box[0], S.nc[0]);
-		const int cy = cell_coord(p.y, S.inv_box[1], S.nc[1]);
-		const int cz = cell_coord(p.z, S.inv_box[2], S.nc[2]);
-		const int R = S.stencil, W = 2 * R + 1, NS = W * W * W;
-		// position inside its cell, for the distance to other cells
-		const float ux = p32.x - cx * S.cell_w[0], uy = p32.y - cy * S.cell_w[1], uz = p32.z - cz * S.cell_w[2];
-		// a cell is culled when its nearest point is farther than r_verlet
-		// by a margin far above the FP32 error of these distances
-		const float cull = (sqrtf(S.rv2f) + 1e-3f) * (sqrtf(S.rv2f) + 1e-3f);
-		auto gap = [](int o, float u, float w) { return o > 0 ? o * w - u : (o < 0 ? u + (-o - 1) * w : 0.f); };
-		auto cell_of = [&](int k, bool &in_range) {
-			const int oz = k / (W * W) - R, oy = (k / W) % W - R, ox = k % W - R;
-			const float gx = gap(ox, ux, S.cell_w[0]), gy = gap(oy, uy, S.cell_w[1]), gz = gap(oz, uz, S.cell_w[2]);
-			in_range = gx * gx + gy * gy + gz * gz <= cull;
-			int z = cz + oz, y = cy + oy, x = cx + ox;
-			z += (z < 0) ? S.nc[2] : (z >= S.nc[2] ? -S.nc[2] : 0);
-			y += (y < 0) ? S.nc[1] : (y >= S.nc[1] ? -S.nc[1] : 0);
-			x += (x < 0) ? S.nc[0] : (x >= S.nc[0] ? -S.nc[0] : 0);
-			return S.cell_first + (z * S.nc[1] + y) * S.nc[0] + x;
-		};
-		if constexpr(K == 32) {
-			// lane l takes cells l, l + 32, ... (1 round for 27 cells, 4 for
-			// 125); the stencil is a compile-time constant of each branch
-			auto stream = [&](auto rounds_tag) {
-				constexpr int ROUNDS = decltype(rounds_tag)::value;
-				int cell[ROUNDS], excl[ROUNDS], base[ROUNDS + 1];
-				base[0] = 0;
-#pragma unroll
-				for(int r = 0; r < ROUNDS; r++) {
-					const int k = l + K * r;
-					int cnt = 0;
-					cell[r] = 0;
-					if(k < NS) {
-						bool in_range;
-						cell[r] = cell_of(k, in_range);
-						if(in_range) cnt = min(count[cell[r]], cap);
-					}
-					int incl = cnt;
-					for(int off = 1; off < K; off <<= 1) {
-						const int v = __shfl_up(incl, off, K);
-						if(l >= off) incl += v;
-					}
-					excl[r] = incl - cnt;
-					base[r + 1] = base[r] + __shfl(incl, K - 1, K);
-				}
-				const int total = base[ROUNDS];
-				for(int m0 = 0; m0 < total; m0 += K) {
-					const int g = m0 + l;
-					int c = 0, slot = 0;
-#pragma unroll
-					for(int r = 0; r < ROUNDS; r++) {
-						// candidates base[r] .. base[r + 1] - 1 come from round r
-						const int gr = g - base[r];
-						int lo = 0;
-						for(int step = K >> 1; step > 0; step >>= 1)
-							if(__shfl(excl[r], lo + step, K) <= gr) lo += step;
-						const int cr = __shfl(cell[r], lo, K), sr = gr - __shfl(excl[r], lo, K);
-						if(g >= base[r] && g < base[r + 1]) {
-							c = cr;
-							slot = sr;
-						}
-					}
-					test(g < total ? items[(size_t) c * cap + slot] : -1, true);
-				}
-			};
-			if(R == 1) stream(std::integral_constant<int, 1>());
-			else stream(std::integral_constant<int, 4>());
-		}
+		const Stencil n = stencil_of(p, p32, S);
+		auto held = [&](int c) { return min(count[c], cap); };
+		if constexpr(K == BUILD_LANES)
+			walk_stencil(n, l, S, held, [&](int c, int slot, int) { test(slot >= 0 ? items[(size_t) c * cap + slot] : -1, true); });
 		else {
-			for(int k = 0; k < NS; k++) {
+			for(int k = 0; k < n.NS; k++) {
 				bool in_range;
-				const int c = cell_of(k, in_range);
-				const int n = in_range ? min(count[c], cap) : 0;
-				for(int m0 = 0; m0 < n; m0 += K) test(m0 + l < n ? items[(size_t) c * cap + m0 + l] : -1, true);
+				const int c = stencil_cell(n, k, S, in_range);
+				const int m = in_range ? held(c) : 0;
+				for(int m0 = 0; m0 < m; m0 += K) test(m0 + l < m ? items[(size_t) c * cap + m0 + l] : -1, true);
 			}
 		}
 	}

@@ -74,6 +74,10 @@ typedef struct oxh_sys {
 	// step (forces of step k use ext_step0 + k), and 1 when any record acts
 	int has_ext;
 	long long ext_step0;
+	// 1 once a list row was longer than the one-launch step sorts in LDS: the
+	// system's rows are built by a launch of their own (last: a checkpoint's
+	// fingerprint ends before it)
+	long long long_rows;
 } oxh_sys;
 
 // One external force acting on one particle (the reference's
@@ -126,7 +130,7 @@ typedef struct oxh_ext_rec {
 typedef struct oxh_sys_state {
 	double K_t, K_r;          // Bussi thermostat internal kinetic energies
 	int need_rebuild;         // skin trigger
-	int error;                // bit 0: FENE bond broken, bit 1: list overflow, bit 2: cell overflow, bit 3: edge-row overflow
+	int error;                // bit 0: FENE bond broken, bit 1: list overflow, bit 2: cell overflow, bit 3: edge-row overflow, bit 5: a row too long for the one-launch step
 	long long n_rebuilds;
 } oxh_sys_state;
 
