@@ -373,6 +373,26 @@ bool fused_ok(const oxh_batch *B) {
 	return b.fuse && !b.edge && b.far_lanes == 0 && b.n_ext == 0 && oxh::fused_lanes(b.lanes);
 }
 
+// whether it could with another launch shape
+bool can_fuse(const oxh_batch *B) {
+	const oxh::Batch &b = B->b;
+	return !B->persist && !b.fp64 && !b.model && !b.cell_build && b.N <= oxh::STEP_MAX_N;
+}
+
+// the second set of buffers of such steps
+oxh_status alloc_step_buffers(oxh_batch *B) {
+	oxh::Batch &b = B->b;
+	const size_t N = b.N;
+	TRY(dalloc(B, &b.pos_alt, N));
+	TRY(dalloc(B, &b.q64_alt, N));
+	TRY(dalloc(B, &b.q32_alt, N));
+	TRY(dalloc(B, &b.bpos_alt, N));
+	TRY(dalloc(B, &b.pos32_alt, N));
+	TRY(dalloc(B, &b.raw_alt, (size_t) std::max(b.ncell_total, 1) * b.cell_cap));
+	TRY(dalloc(B, &b.step_need, 3 * (size_t) (b.nsys + 1)));
+	return OXH_OK;
+}
+
 // what is the same for every step of a chunk
 oxh::StepArgs step_args(const oxh_batch *B) {
 	const oxh::Batch &b = B->b;
@@ -1707,20 +1727,11 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 		const char *e = getenv("OXH_EDGE");
 		if(!B->pool && !B->persist && !b.fp64 && !b.model && !(e && atoi(e) == 0)) TRYB(alloc_edges(B, std::min(b.max_neigh, 64)));
 	}
-	// one launch per MD step: the second set of buffers (OXH_FUSE=0 keeps
-	// one kernel per phase)
+	// one launch per MD step (OXH_FUSE=0 keeps one kernel per phase)
 	{
 		const char *e = getenv("OXH_FUSE");
-		if(!B->persist && !b.fp64 && !b.model && !b.cell_build && N <= oxh::STEP_MAX_N && !(e && atoi(e) == 0)) {
-			TRYB(dalloc(B, &b.pos_alt, N));
-			TRYB(dalloc(B, &b.q64_alt, N));
-			TRYB(dalloc(B, &b.q32_alt, N));
-			TRYB(dalloc(B, &b.bpos_alt, N));
-			TRYB(dalloc(B, &b.pos32_alt, N));
-			TRYB(dalloc(B, &b.raw_alt, (size_t) std::max(ncell, 1) * b.cell_cap));
-			TRYB(dalloc(B, &b.step_need, 3 * (size_t) (n_sys + 1)));
-			b.fuse = true;
-		}
+		b.fuse = can_fuse(B) && !(e && atoi(e) == 0);
+		if(b.fuse) TRYB(alloc_step_buffers(B));
 	}
 	// far pairs kept by their backbone sites: grid-engine batches and
 	// pools, systems with cells in boxes wide enough that backbone sites
@@ -2925,12 +2936,18 @@ struct CheckpointHeader {
 	char magic[8];            // "OXHCKPT2"
 	int N, nsys, fp64, persist;
 	long long step, since_sort, since_fix;
-	int lanes, force_block, far_lanes, far_block, edge, edge_group, ecap, pad_;
+	int lanes, force_block, far_lanes, far_block, edge, edge_group, ecap;
+	// CKPT_*; 0 in files of before there was a choice, which restore into
+	// whatever the batch has
+	int form;
 	// FNV-1a of every system's parameters (range, box, cells, model
 	// constants, integrator, thermostat and seed): a checkpoint restores
 	// only into a batch built from the same systems
 	unsigned long long sys_hash;
 };
+
+// CheckpointHeader::form: the field is set; packed close pairs; one launch per step
+constexpr int CKPT_FORM = 1, CKPT_PACK = 2, CKPT_FUSE = 4;
 
 unsigned long long systems_fingerprint(const oxh_batch *B) {
 	unsigned long long h = 1469598103934665603ull;
@@ -3001,6 +3018,7 @@ oxh_status oxh_batch_save(oxh_batch *B, void *buf, size_t bytes) {
 	h.edge = b.edge;
 	h.edge_group = b.edge_group;
 	h.ecap = b.ecap;
+	h.form = CKPT_FORM | (b.pack ? CKPT_PACK : 0) | (b.fuse ? CKPT_FUSE : 0);
 	char *p = (char *) buf;
 	std::memcpy(p, &h, sizeof(h));
 	p += sizeof(h);
@@ -3035,6 +3053,11 @@ oxh_status oxh_batch_restore(oxh_batch *B, const void *buf, size_t bytes) {
 	b.far_block = h.far_block;
 	b.edge = h.edge;
 	b.edge_group = h.edge_group;
+	if(h.form & CKPT_FORM) {
+		b.pack = (h.form & CKPT_PACK) != 0;
+		b.fuse = (h.form & CKPT_FUSE) != 0 && can_fuse(B);
+		if(b.fuse && !b.step_need) TRY(alloc_step_buffers(B));
+	}
 	const char *p = (const char *) buf + sizeof(h);
 	for(auto &x : ckpt_layout(B)) {
 		HIPCHK(hipMemcpyAsync(x.first, p, x.second, hipMemcpyHostToDevice, b.stream));
