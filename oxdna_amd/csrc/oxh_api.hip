@@ -379,18 +379,49 @@ bool can_fuse(const oxh_batch *B) {
 	return !B->persist && !b.fp64 && !b.model && !b.cell_build && b.N <= oxh::STEP_MAX_N;
 }
 
-// the second set of buffers of such steps
+// the second set of buffers of such steps (128 B per nucleotide, and the
+// cells' slots): held while steps use it, and given back by batches whose
+// shape, or whose external forces, keep one kernel per phase
+oxh_status free_step_buffers(oxh_batch *B) {
+	oxh::Batch &b = B->b;
+	HIPCHK(hipStreamSynchronize(b.stream));
+	const size_t N = b.N, slots = (size_t) std::max(b.ncell_total, 1) * b.cell_cap;
+	auto give = [&](auto *&p, size_t count) {
+		if(!p) return;
+		(void) hipFree(p);
+		B->device_bytes -= count * sizeof(*p);
+		p = nullptr;
+	};
+	give(b.pos_alt, N);
+	give(b.q64_alt, N);
+	give(b.q32_alt, N);
+	give(b.bpos_alt, N);
+	give(b.pos32_alt, N);
+	give(b.raw_alt, slots);
+	give(b.step_need, 3 * (size_t) (b.nsys + 1));
+	return OXH_OK;
+}
+
 oxh_status alloc_step_buffers(oxh_batch *B) {
 	oxh::Batch &b = B->b;
-	const size_t N = b.N;
-	TRY(dalloc(B, &b.pos_alt, N));
-	TRY(dalloc(B, &b.q64_alt, N));
-	TRY(dalloc(B, &b.q32_alt, N));
-	TRY(dalloc(B, &b.bpos_alt, N));
-	TRY(dalloc(B, &b.pos32_alt, N));
-	TRY(dalloc(B, &b.raw_alt, (size_t) std::max(b.ncell_total, 1) * b.cell_cap));
-	TRY(dalloc(B, &b.step_need, 3 * (size_t) (b.nsys + 1)));
-	return OXH_OK;
+	if(b.step_need) return OXH_OK;
+	const size_t N = b.N, slots = (size_t) std::max(b.ncell_total, 1) * b.cell_cap;
+	auto all = [&]() -> oxh_status {
+		TRY(dalloc(B, &b.pos_alt, N));
+		TRY(dalloc(B, &b.q64_alt, N));
+		TRY(dalloc(B, &b.q32_alt, N));
+		TRY(dalloc(B, &b.bpos_alt, N));
+		TRY(dalloc(B, &b.pos32_alt, N));
+		TRY(dalloc(B, &b.raw_alt, slots));
+		return dalloc(B, &b.step_need, 3 * (size_t) (b.nsys + 1));
+	};
+	const oxh_status s = all();
+	if(s != OXH_OK) {
+		const std::string msg = g_err;
+		(void) free_step_buffers(B);
+		g_err = msg;
+	}
+	return s;
 }
 
 // what is the same for every step of a chunk
@@ -1774,6 +1805,7 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 		b.far_lanes = 0;
 		if(const char *f = getenv("OXH_FAR_LANES")) b.far_lanes = atoi(f);
 	}
+	if(!fused_ok(B)) TRYB(free_step_buffers(B));
 	// graph chunk: enough steps to amortise the launch, at most ~2k kernels
 	B->chunk = 64;
 	if(const char *g = getenv("OXH_GRAPH")) B->use_graph = atoi(g) != 0;
@@ -1958,6 +1990,7 @@ oxh_status oxh_batch_run(oxh_batch *B, long long n_steps) {
 	if(n_steps < 0) return fail(OXH_ERR_ARG, "negative step count");
 	oxh::Batch &b = B->b;
 	HIPCHK(hipSetDevice(b.device));
+	if(fused_ok(B)) TRY(alloc_step_buffers(B));
 	long long done = 0;
 	int retries = 0;
 	while(done < n_steps) {
@@ -2507,6 +2540,7 @@ oxh_status oxh_batch_set_external_forces(oxh_batch *B, int sys, int n, const oxh
 		(void) hipGraphExecDestroy(b.graph_exec);
 		b.graph_exec = nullptr;
 	}
+	if(!fused_ok(B)) TRY(free_step_buffers(B));
 	k_clear_err<<<(b.nsys + 63) / 64, 64, 0, b.stream>>>(b.nsys, b.d_state, oxh::ERR_EXT);
 	enqueue_forces(B);
 	std::vector<oxh_sys_state> st;
@@ -3056,7 +3090,7 @@ oxh_status oxh_batch_restore(oxh_batch *B, const void *buf, size_t bytes) {
 	if(h.form & CKPT_FORM) {
 		b.pack = (h.form & CKPT_PACK) != 0;
 		b.fuse = (h.form & CKPT_FUSE) != 0 && can_fuse(B);
-		if(b.fuse && !b.step_need) TRY(alloc_step_buffers(B));
+		if(fused_ok(B)) TRY(alloc_step_buffers(B));
 	}
 	const char *p = (const char *) buf + sizeof(h);
 	for(auto &x : ckpt_layout(B)) {

@@ -84,3 +84,37 @@ def test_paths_that_are_not_one_launch(hip, monkeypatch):
         assert b.routes()["one_launch"]
         b.set_external_forces([dict(type="trap", particle=0, stiff=1.0, pos0=s.pos[0], dir=(0.0, 0.0, 1.0))])
         assert not b.routes()["one_launch"]
+
+
+def test_second_buffers_only_while_steps_use_them(hip, monkeypatch):
+    """Device bytes held, against a batch that never takes one launch per step."""
+    s = _gas(3, 100, 20)
+    monkeypatch.setenv("OXH_FORCE_LANES", "8")
+
+    def held(fuse, far):
+        monkeypatch.setenv("OXH_FUSE", str(fuse))
+        monkeypatch.setenv("OXH_FAR_LANES", str(far))
+        return hip.HIPBatch(s, dt=0.003, verlet_skin=0.05, seed=3, **THERMO["langevin"])
+
+    with held(0, 0) as b:
+        base = b.stats()["device_bytes"]
+        b.run(120)
+        want = _final(b, 0)
+    with held(1, 8) as b:
+        assert b.stats()["device_bytes"] == base
+    with held(1, 0) as b:
+        used = b.stats()["device_bytes"]
+        assert used >= base + 112 * s.N
+        b.run(40)
+        ck = b.checkpoint()
+        b.set_external_forces([dict(type="trap", particle=0, stiff=1.0, pos0=s.pos[0], dir=(0.0, 0.0, 1.0))])
+        less = b.stats()["device_bytes"]
+        assert less < used - 112 * s.N
+        b.run(10)
+        b.set_external_forces([])
+        b.restore(ck)
+        b.run(80)
+        assert b.routes()["one_launch"] and b.stats()["device_bytes"] >= used
+        got = _final(b, 0)
+    for key in KEYS:
+        assert np.array_equal(want[key], got[key]), key
