@@ -92,8 +92,8 @@ __device__ __forceinline__ void build_row_binned(int i, int l, int s, const Step
 				full |= held > a.cell_cap;
 				return min(held, a.cell_cap);
 			},
-			[&](int c, int slot, int kc) {
-				const int j = slot >= 0 ? a.raw[(size_t) c * a.cell_cap + slot] : -1;
+			[&](bool have, int c, int slot, int kc) {
+				const int j = have ? a.raw[(size_t) c * a.cell_cap + slot] : -1;
 				bool close, far;
 				cand.test(j, close, far);
 				const uint64_t bc = __ballot(close) & gmask, bf = __ballot(far) & gmask;

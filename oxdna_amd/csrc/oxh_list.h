@@ -122,9 +122,9 @@ __device__ __forceinline__ int stencil_cell(const Stencil &n, int k, const oxh_s
 }
 
 // The candidates of a particle of a system with cells, in chunks of one per
-// lane (the 32 lanes of a group call it): test(cell, slot, k) with the
+// lane (the 32 lanes of a group call it): test(have, cell, slot, k) with the
 // candidates in the order of the stencil's cells k, then of their slots
-// (slot < 0: none for this lane).  held(cell) is a cell's occupancy.  Lane l
+// (have: there is one for this lane).  held(cell) is a cell's occupancy.  Lane l
 // takes cells l, l + 32, ... (1 round for 27 cells, 4 for 125); lane prefix
 // sums of the occupancies number the candidates, and each lane finds its
 // candidate's cell by a binary search over them: the cells' loads overlap
@@ -158,7 +158,7 @@ __device__ __forceinline__ void walk_stencil(const Stencil &n, int l, const oxh_
 		const int total = base[ROUNDS];
 		for(int m0 = 0; m0 < total; m0 += K) {
 			const int g = m0 + l;
-			int c = 0, slot = -1, kc = 0;
+			int c = 0, slot = 0, kc = 0;
 #pragma unroll
 			for(int r = 0; r < ROUNDS; r++) {
 				// candidates base[r] .. base[r + 1] - 1 come from round r
@@ -173,7 +173,7 @@ __device__ __forceinline__ void walk_stencil(const Stencil &n, int l, const oxh_
 					kc = lo + K * r;
 				}
 			}
-			test(c, slot, kc);
+			test(g < total, c, slot, kc);
 		}
 	};
 	if(n.R == 1) stream(std::integral_constant<int, 1>());
@@ -234,7 +234,7 @@ __device__ __forceinline__ void build_row(int i, int l, int s, const double4 *__
 		const Stencil n = stencil_of(p, p32, S);
 		auto held = [&](int c) { return min(count[c], cap); };
 		if constexpr(K == BUILD_LANES)
-			walk_stencil(n, l, S, held, [&](int c, int slot, int) { test(slot >= 0 ? items[(size_t) c * cap + slot] : -1, true); });
+			walk_stencil(n, l, S, held, [&](bool have, int c, int slot, int) { test(have ? items[(size_t) c * cap + slot] : -1, true); });
 		else {
 			for(int k = 0; k < n.NS; k++) {
 				bool in_range;
