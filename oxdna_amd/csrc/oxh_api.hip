@@ -65,6 +65,8 @@ struct oxh_batch {
 	// the rebuild flag of a force call on the caller's buffers, or whether a
 	// chunk of steps left an error bit
 	int *h_flag = nullptr;
+	// force calls on the caller's buffers in a row, up to 2, that needed lists
+	int rebuilt_calls = 0;
 	// what the host reads: page-locked staging (two halves), and the device
 	// buffer of what does not fit in STAGE_DIRECT
 	std::mutex stage_mutex;
@@ -1943,21 +1945,31 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *B, const double *d_pos, con
 	const int bs = 256, g = (b.N + bs - 1) / bs;
 	k_load_caller_state<<<g, bs, 0, st>>>(b.N, (const double4 *) d_pos, (const double4 *) d_quat, b.orig, b.pinfo, b.bonds, b.d_sys,
 			b.rlist, b.pos, b.q64, b.q32, b.bpos, b.back64, b.d_state, b.any_rebuild, b.blist);
+	auto forces = [&](int k) {
+		if(B->persist) oxh::launch_persist_forces(st, b, false, B->persist_block, k);
+		else oxh::launch_forces(st, b, false, k);
+	};
 	// Most calls need no list: the forces and the additions follow at once,
 	// on the lists in hand, and both do nothing when the state just loaded
 	// asks for a rebuild.  The host learns which from the additions' word,
 	// so that a call is the state, the forces, the additions and one wait
 	// (24,576-nt gas: 106 us with the list kernels and a copy back queued in
-	// every call, 51 us without).
-	auto forces = [&](int k) {
-		if(B->persist) oxh::launch_persist_forces(st, b, false, B->persist_block);
-		else oxh::launch_forces(st, b, false, k);
-	};
-	forces(oxh::K_IF_LISTS_HOLD);
-	launch_add(b, st, d_forces, d_torques, b.any_rebuild, nullptr, 0, B->h_flag);
-	HIPCHK(hipGetLastError());
-	HIPCHK(hipStreamSynchronize(st));
-	if(*(volatile int *) B->h_flag == 0) return OXH_OK;
+	// every call, 51 us without).  A caller whose last two calls both needed
+	// lists, which successive states of an MD run do not, moves its states
+	// further than the skin every time: without cells its list kernels are
+	// queued at once (a call of 40 nt that rebuilds 77 -> 50 us, of 320 nt
+	// 220 -> 126, of 777 nt 70 -> 55).  With cells that measured slower than
+	// the first try and its wait (4,800 nt 83 -> 92 us, 98,304 nt 206 -> 214).
+	if(B->rebuilt_calls < 2 || b.any_cells) {
+		forces(oxh::K_IF_LISTS_HOLD);
+		launch_add(b, st, d_forces, d_torques, b.any_rebuild, nullptr, 0, B->h_flag);
+		HIPCHK(hipGetLastError());
+		HIPCHK(hipStreamSynchronize(st));
+		if(*(volatile int *) B->h_flag == 0) {
+			B->rebuilt_calls = 0;
+			return OXH_OK;
+		}
+	}
 	std::vector<oxh_sys_state> sst(b.nsys);
 	for(int attempt = 0;; attempt++) {
 		if(attempt == 12) return fail(OXH_ERR_SYSTEM, "neighbour list keeps overflowing");
@@ -1972,6 +1984,9 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *B, const double *d_pos, con
 		bool overflow = false;
 		for(auto &x : sst) overflow |= (x.error & oxh::ERR_OVERFLOW) != 0;
 		if(!overflow) {
+			bool any = attempt > 0;
+			for(auto &x : sst) any |= x.need_rebuild != 0;
+			B->rebuilt_calls = any ? std::min(B->rebuilt_calls + 1, 2) : 0;
 			// the systems rebuilt count one list build each, as in a step
 			k_count_rebuilds<<<(b.nsys + 63) / 64, 64, 0, st>>>(b.nsys, b.d_state, b.any_rebuild);
 			break;

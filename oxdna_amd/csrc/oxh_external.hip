@@ -420,8 +420,9 @@ template<class FT>
 __global__ void k_ext_forces(int N, const double4 *__restrict__ pos, const int4 *__restrict__ img, const int *__restrict__ orig,
 		const int2 *__restrict__ pinfo, const oxh_sys *__restrict__ systems, const long long *__restrict__ pstep,
 		const int *__restrict__ slot_of, const int *__restrict__ ext_off, const oxh_ext_rec *__restrict__ rec, const double *__restrict__ com,
-		oxh_sys_state *__restrict__ state, FT *__restrict__ F) {
+		oxh_sys_state *__restrict__ state, FT *__restrict__ F, int k_step, const int *__restrict__ any) {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if(k_step == K_IF_LISTS_HOLD && *any) return;
 	if(i >= N) return;
 	const int s = pinfo[i].y;
 	const oxh_sys &S = systems[s];
@@ -458,17 +459,17 @@ __global__ void k_slot_of(int N, const int *__restrict__ orig, const int2 *__res
 
 }  // namespace
 
-void launch_ext_forces(hipStream_t st, const Batch &b) {
+void launch_ext_forces(hipStream_t st, const Batch &b, int k) {
 	if(b.n_ext == 0 || b.N == 0) return;
 	if(b.n_grp > 0)
 		k_ext_groups<<<b.n_grp, 256, 0, st>>>(b.n_grp, b.ext_grp, b.ext_grp_sys, b.ext_idx, b.pos, b.img, b.slot_of, b.d_sys, b.ext_com);
 	const int bs = 256, g = (b.N + bs - 1) / bs;
 	if(b.fp64)
 		k_ext_forces<double4><<<g, bs, 0, st>>>(b.N, b.pos, b.img, b.orig, b.pinfo, b.d_sys, b.pstep, b.slot_of, b.ext_off, b.ext_rec,
-				b.ext_com, b.d_state, b.F64);
+				b.ext_com, b.d_state, b.F64, k, b.any_rebuild);
 	else
 		k_ext_forces<float4><<<g, bs, 0, st>>>(b.N, b.pos, b.img, b.orig, b.pinfo, b.d_sys, b.pstep, b.slot_of, b.ext_off, b.ext_rec,
-				b.ext_com, b.d_state, b.F);
+				b.ext_com, b.d_state, b.F, k, b.any_rebuild);
 }
 
 void launch_slot_of(hipStream_t st, const Batch &b) {

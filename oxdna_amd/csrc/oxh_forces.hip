@@ -95,6 +95,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 	static_assert(P >= 1 && P <= 64 && (64 % P) == 0, "P must divide the wave");
 	const int lane = threadIdx.x & 63;
 	const int i0 = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * P;
+	if(k == K_IF_LISTS_HOLD && *any) return;
 	if(k >= 0 && blockIdx.x == 0 && threadIdx.x == 0) *any = 0;
 	if(i0 >= N) return;   // whole waves
 	const int ii = i0 + lane;
@@ -164,7 +165,8 @@ __global__ void __launch_bounds__(256) k_edge_gather(int N, const double4 *__res
 		const int *__restrict__ nbr, const int2 *__restrict__ nnbr, int max_neigh, const oxh_sys *__restrict__ systems,
 		const int *__restrict__ ein, const int2 *__restrict__ ecount, int ecap, const float4 *__restrict__ E1, const float4 *__restrict__ E2,
 		const float4 *__restrict__ E3, const float4 *__restrict__ B1, const float4 *__restrict__ B2, const float4 *__restrict__ B3,
-		float4 *__restrict__ Fout, float4 *__restrict__ Tout) {
+		float4 *__restrict__ Fout, float4 *__restrict__ Tout, int k_step, const int *__restrict__ any) {
+	if(k_step == K_IF_LISTS_HOLD && *any) return;
 	const int t = blockIdx.x * blockDim.x + threadIdx.x;
 	const int i = t / K;
 	const int l = t % K;
@@ -255,9 +257,11 @@ template<int K, bool SPLIT, bool SMALL>
 __global__ void __launch_bounds__(256) k_forces_far(int N, const double4 *__restrict__ pos, const float4 *__restrict__ q32,
 		const float4 *__restrict__ bpos, const int *__restrict__ nbr, const int2 *__restrict__ nnbr, int max_neigh,
 		const int2 *__restrict__ pinfo, const oxh_sys *__restrict__ systems, float4 *__restrict__ Fio, float4 *__restrict__ Tio,
-		double *__restrict__ esplit, int k_step, const int *__restrict__ limit, double *__restrict__ stress, int xcd) {
+		double *__restrict__ esplit, int k_step, const int *__restrict__ limit, const int *__restrict__ any, double *__restrict__ stress,
+		int xcd) {
 	const int blk = xcd ? xcd_block(((unsigned) N * K + blockDim.x - 1) / blockDim.x) : (int) blockIdx.x;
 	if(blk < 0) return;
+	if(k_step == K_IF_LISTS_HOLD && *any) return;
 	const int t = blk * blockDim.x + threadIdx.x;
 	const int i = t / K;
 	const int l = t % K;
@@ -370,9 +374,11 @@ template<int K, bool SPLIT>
 __global__ void __launch_bounds__(256) k_forces_far_dp(int N, const double4 *__restrict__ pos, const double4 *__restrict__ q64,
 		const double4 *__restrict__ back64, const float4 *__restrict__ bpos, const int *__restrict__ nbr, const int2 *__restrict__ nnbr, int max_neigh,
 		const int2 *__restrict__ pinfo, const oxh_sys *__restrict__ systems, double4 *__restrict__ Fio, double4 *__restrict__ Tio,
-		double *__restrict__ esplit, int k_step, const int *__restrict__ limit, double *__restrict__ stress, int xcd) {
+		double *__restrict__ esplit, int k_step, const int *__restrict__ limit, const int *__restrict__ any, double *__restrict__ stress,
+		int xcd) {
 	const int blk = xcd ? xcd_block(((unsigned) N * K + blockDim.x - 1) / blockDim.x) : (int) blockIdx.x;
 	if(blk < 0) return;
+	if(k_step == K_IF_LISTS_HOLD && *any) return;
 	const int t = blk * blockDim.x + threadIdx.x;
 	const int i = t / K;
 	const int l = t % K;
@@ -448,10 +454,10 @@ static void launch_far_dp(hipStream_t st, const Batch &b, bool split, int k) {
 	const int *lim = k >= 0 ? b.limit : nullptr;
 	if(split)
 		k_forces_far_dp<K, true><<<grid, block, 0, st>>>(b.N, b.pos, b.q64, b.back64, b.bpos, b.nbr, b.nnbr, b.max_neigh, b.pinfo, b.d_sys, b.F64,
-				b.T64, b.esplit, k, lim, b.stress, b.xcd);
+				b.T64, b.esplit, k, lim, b.any_rebuild, b.stress, b.xcd);
 	else
 		k_forces_far_dp<K, false><<<grid, block, 0, st>>>(b.N, b.pos, b.q64, b.back64, b.bpos, b.nbr, b.nnbr, b.max_neigh, b.pinfo, b.d_sys, b.F64,
-				b.T64, nullptr, k, lim, nullptr, b.xcd);
+				b.T64, nullptr, k, lim, b.any_rebuild, nullptr, b.xcd);
 }
 
 // all-FP64 forces: close (+ bonded) kernel with b.lanes, far pairs inline
@@ -509,10 +515,10 @@ static void launch_far_k(hipStream_t st, const Batch &b, bool split, int block, 
 	dim3 grid(b.xcd ? xcd_grid(nblk) : nblk);
 	if(split)
 		k_forces_far<K, true, SMALL><<<grid, block, 0, st>>>(b.N, b.pos, b.q32, b.bpos, b.nbr, b.nnbr, b.max_neigh, b.pinfo, b.d_sys, b.F,
-				b.T, b.esplit, k, k >= 0 ? b.limit : nullptr, b.stress, b.xcd);
+				b.T, b.esplit, k, k >= 0 ? b.limit : nullptr, b.any_rebuild, b.stress, b.xcd);
 	else
 		k_forces_far<K, false, SMALL><<<grid, block, 0, st>>>(b.N, b.pos, b.q32, b.bpos, b.nbr, b.nnbr, b.max_neigh, b.pinfo, b.d_sys, b.F,
-				b.T, nullptr, k, k >= 0 ? b.limit : nullptr, nullptr, b.xcd);
+				b.T, nullptr, k, k >= 0 ? b.limit : nullptr, b.any_rebuild, nullptr, b.xcd);
 }
 
 // slot pools take any system later, so they keep the small-box path
@@ -533,14 +539,14 @@ static void launch_edge_pairs(hipStream_t st, const Batch &b, int k) {
 }
 
 template<int K>
-static void launch_edge_gather(hipStream_t st, const Batch &b, bool far_inline) {
+static void launch_edge_gather(hipStream_t st, const Batch &b, bool far_inline, int k) {
 	dim3 grid((unsigned) (((size_t) b.N * K + 255) / 256));
 	if(far_inline)
 		k_edge_gather<K, true><<<grid, 256, 0, st>>>(b.N, b.pos, b.q64, b.q32, b.bpos, b.bonds, b.pinfo, b.nbr, b.nnbr, b.max_neigh, b.d_sys,
-				b.ein, b.ecount, b.ecap, b.E1, b.E2, b.E3, b.B1, b.B2, b.B3, b.F, b.T);
+				b.ein, b.ecount, b.ecap, b.E1, b.E2, b.E3, b.B1, b.B2, b.B3, b.F, b.T, k, b.any_rebuild);
 	else
 		k_edge_gather<K, false><<<grid, 256, 0, st>>>(b.N, b.pos, b.q64, b.q32, b.bpos, b.bonds, b.pinfo, b.nbr, b.nnbr, b.max_neigh, b.d_sys,
-				b.ein, b.ecount, b.ecap, b.E1, b.E2, b.E3, b.B1, b.B2, b.B3, b.F, b.T);
+				b.ein, b.ecount, b.ecap, b.E1, b.E2, b.E3, b.B1, b.B2, b.B3, b.F, b.T, k, b.any_rebuild);
 }
 
 // half-list form: b.edge_group particles per wave in the pair kernel,
@@ -554,12 +560,12 @@ static void launch_edge(hipStream_t st, const Batch &b, bool far_inline, int k) 
 	default: launch_edge_pairs<16>(st, b, k); break;
 	}
 	switch(b.lanes) {
-	case 1: launch_edge_gather<1>(st, b, far_inline); break;
-	case 2: launch_edge_gather<2>(st, b, far_inline); break;
-	case 4: launch_edge_gather<4>(st, b, far_inline); break;
-	case 16: launch_edge_gather<16>(st, b, far_inline); break;
-	case 32: launch_edge_gather<32>(st, b, far_inline); break;
-	default: launch_edge_gather<8>(st, b, far_inline); break;
+	case 1: launch_edge_gather<1>(st, b, far_inline, k); break;
+	case 2: launch_edge_gather<2>(st, b, far_inline, k); break;
+	case 4: launch_edge_gather<4>(st, b, far_inline, k); break;
+	case 16: launch_edge_gather<16>(st, b, far_inline, k); break;
+	case 32: launch_edge_gather<32>(st, b, far_inline, k); break;
+	default: launch_edge_gather<8>(st, b, far_inline, k); break;
 	}
 }
 
@@ -616,7 +622,7 @@ void launch_pair_forces(hipStream_t st, const Batch &b, bool split, int k) {
 // on top
 void launch_forces(hipStream_t st, const Batch &b, bool split, int k) {
 	launch_pair_forces(st, b, split, k);
-	launch_ext_forces(st, b);
+	launch_ext_forces(st, b, k);
 }
 
 }  // namespace oxh

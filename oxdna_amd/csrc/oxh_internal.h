@@ -174,13 +174,13 @@ size_t persist_lds_bytes(int nmax);
 // largest system the LDS-resident engine takes: its dynamic LDS plus the
 // engine's static LDS within 64 KiB per workgroup
 constexpr int PERSIST_LDS_MAX_N = 80;
-void launch_persist_forces(hipStream_t st, const Batch &b, bool split, int block);
 
 // k = index of the step inside the current chunk (checked against limit);
 // k < 0: forces of every system's current state, whatever its limit
 // (K_IF_LISTS_HOLD: nothing while *any_rebuild is set)
 constexpr int K_IF_LISTS_HOLD = -2;
 void launch_forces(hipStream_t st, const Batch &b, bool split, int k = -1);
+void launch_persist_forces(hipStream_t st, const Batch &b, bool split, int block, int k = -1);
 // list builds read positions from src (the current positions, or rlist to
 // rebuild exactly the lists of the last build)
 void launch_cells(hipStream_t st, const Batch &b, const double4 *src);
@@ -231,7 +231,7 @@ void launch_refresh_vel(hipStream_t st, const Batch &b, int i0, int n);
 void launch_prepare_mirror(hipStream_t st, const Batch &b);
 int launch_hilbert_sort(hipStream_t st, Batch &b);
 // adds every particle's external forces to F (F64) of the current state
-void launch_ext_forces(hipStream_t st, const Batch &b);
+void launch_ext_forces(hipStream_t st, const Batch &b, int k);
 // slot_of from orig (after an upload or a sort)
 void launch_slot_of(hipStream_t st, const Batch &b);
 // oxRNA / oxRNA2 pair forces (written, not accumulated) into F / T, or

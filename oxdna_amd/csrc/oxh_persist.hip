@@ -275,7 +275,8 @@ __global__ void __launch_bounds__(BLOCK) k_persist_lds(PersistArgs a, int nmax) 
 // nucleotide (after uploads, list rebuilds and for observables), so that
 // runs continue from exactly the forces the engine itself computes.
 template<bool SPLIT, int BLOCK>
-__global__ void __launch_bounds__(BLOCK) k_persist_forces(PersistArgs a, double *esplit, double *stress) {
+__global__ void __launch_bounds__(BLOCK) k_persist_forces(PersistArgs a, double *esplit, double *stress, const int *hold) {
+	if(hold && *hold) return;
 	const oxh_sys &S = a.systems[blockIdx.x];
 	const int K = persist_lanes(S.n, BLOCK);
 	const int tid = threadIdx.x;
@@ -334,16 +335,17 @@ void launch_persist(hipStream_t st, const Batch &b, int nsteps, int block) {
 	else k_persist<512><<<b.nsys, 512, 0, st>>>(make_args(b, nsteps));
 }
 
-void launch_persist_forces(hipStream_t st, const Batch &b, bool split, int block) {
+void launch_persist_forces(hipStream_t st, const Batch &b, bool split, int block, int k) {
 	if(b.N == 0) return;
+	const int *hold = k == K_IF_LISTS_HOLD ? b.any_rebuild : nullptr;
 	PersistArgs a = make_args(b, 0);
 	if(block == 256) {
-		if(split) k_persist_forces<true, 256><<<b.nsys, 256, 0, st>>>(a, b.esplit, b.stress);
-		else k_persist_forces<false, 256><<<b.nsys, 256, 0, st>>>(a, nullptr, nullptr);
+		if(split) k_persist_forces<true, 256><<<b.nsys, 256, 0, st>>>(a, b.esplit, b.stress, hold);
+		else k_persist_forces<false, 256><<<b.nsys, 256, 0, st>>>(a, nullptr, nullptr, hold);
 	}
 	else {
-		if(split) k_persist_forces<true, 512><<<b.nsys, 512, 0, st>>>(a, b.esplit, b.stress);
-		else k_persist_forces<false, 512><<<b.nsys, 512, 0, st>>>(a, nullptr, nullptr);
+		if(split) k_persist_forces<true, 512><<<b.nsys, 512, 0, st>>>(a, b.esplit, b.stress, hold);
+		else k_persist_forces<false, 512><<<b.nsys, 512, 0, st>>>(a, nullptr, nullptr, hold);
 	}
 }
 
