@@ -490,8 +490,10 @@ oxh_status oxh_batch_stats(oxh_batch *b, double *out12);
  * integration in one kernel: grid-engine batches and pools of the mixed
  * oxDNA2 form with the far pairs inline, lists built per particle and no
  * external forces; systems with rows above 512 entries have theirs built by a
- * launch of their own before it), else 0. */
-oxh_status oxh_batch_routes(oxh_batch *b, int *out1);
+ * launch of their own before it), else 0; out[1] threads per nucleotide of the
+ * far-pair kernel of oxh_interaction_compute_forces (0 = inline), which is
+ * timed apart from the steps'. */
+oxh_status oxh_batch_routes(oxh_batch *b, int *out2);
 
 /* Average duration in ms of n back-to-back launches of the force kernel on
  * the batch's stream, timed with HIP events (the reference times its steps

@@ -373,9 +373,9 @@ class HIPBatch:
     def routes(self) -> dict:
         """Which kernels the batch's work takes as it stands
         (oxh_batch_routes)."""
-        out = np.zeros(1, np.int32)
+        out = np.zeros(2, np.int32)
         check(lib().oxh_batch_routes(self.h, ptr(out)), "oxh_batch_routes")
-        return dict(one_launch=bool(out[0]))
+        return dict(one_launch=bool(out[0]), call_far_lanes=int(out[1]))
 
 
 class HIPPool(HIPBatch):

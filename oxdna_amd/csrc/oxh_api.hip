@@ -67,6 +67,9 @@ struct oxh_batch {
 	int *h_flag = nullptr;
 	// force calls on the caller's buffers in a row, up to 2, that needed lists
 	int rebuilt_calls = 0;
+	// far-pair kernel of those calls where steps take the far pairs inline
+	// (0: inline too)
+	int call_far_lanes = 0, call_far_block = 256;
 	// what the host reads: page-locked staging (two halves), and the device
 	// buffer of what does not fit in STAGE_DIRECT
 	std::mutex stage_mutex;
@@ -1240,19 +1243,20 @@ oxh_status autotune_forces(oxh_batch *B) {
 		if(fused_ok(B)) oxh::launch_step(b.stream, sa, b.lanes, b.pack, b.force_block, 0, false);
 		else oxh::launch_forces(b.stream, b, false);
 	};
-	auto timeit = [&](float &ms) -> oxh_status {
-		const bool brief = fused_ok(B) && b.N < 16384;
+	auto time_of = [&](float &ms, bool brief, auto &&launch) -> oxh_status {
 		const int reps = brief ? 8 : 3;
-		evaluate();
+		launch();
 		if(brief) k_lead<<<1, 64, 0, b.stream>>>();
 		HIPCHK(hipEventRecord(e0, b.stream));
-		for(int k = 0; k < reps; k++) evaluate();
+		for(int k = 0; k < reps; k++) launch();
 		HIPCHK(hipEventRecord(e1, b.stream));
 		HIPCHK(hipEventSynchronize(e1));
 		HIPCHK(hipEventElapsedTime(&ms, e0, e1));
 		ms /= reps;
 		return OXH_OK;
 	};
+	auto timeit = [&](float &ms) { return time_of(ms, fused_ok(B) && b.N < 16384, evaluate); };
+	auto time_call = [&](float &ms) { return time_of(ms, true, [&]() { oxh::launch_forces(b.stream, b, false); }); };
 	const int lanes[] = {1, 2, 4, 8, 16, 32};
 	const int blocks[] = {64, 128, 256};
 	float best = 1e30f;
@@ -1386,6 +1390,19 @@ oxh_status autotune_forces(oxh_batch *B) {
 				}
 			}
 	if(bfl != 0 && inline_best <= best + margin) {
+		// a force call on the caller's buffers has no such launches to save:
+		// it takes the far kernel if that wins by itself (24 bundles of 960 nt
+		// at salt 0.1, a call: inline 147 us, with the far kernel 138)
+		float one, two;
+		b.far_lanes = bfl;
+		b.far_block = bfb;
+		TRY(time_call(two));
+		b.far_lanes = 0;
+		TRY(time_call(one));
+		if(two < 0.98f * one) {
+			B->call_far_lanes = bfl;
+			B->call_far_block = bfb;
+		}
 		best = inline_best;
 		bfl = 0;
 	}
@@ -1942,6 +1959,19 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *B, const double *d_pos, con
 	hipStream_t st = stream ? (hipStream_t) stream : b.stream;
 	// work queued on the batch's own stream comes first
 	if(st != b.stream) HIPCHK(hipStreamSynchronize(b.stream));
+	// the far pairs in the calls' own shape
+	struct FarShape {
+		oxh::Batch &b;
+		const int lanes, block;
+		~FarShape() {
+			b.far_lanes = lanes;
+			b.far_block = block;
+		}
+	} steps = {b, b.far_lanes, b.far_block};
+	if(B->call_far_lanes > 0 && b.far_lanes == 0 && !b.edge) {
+		b.far_lanes = B->call_far_lanes;
+		b.far_block = B->call_far_block;
+	}
 	const int bs = 256, g = (b.N + bs - 1) / bs;
 	k_load_caller_state<<<g, bs, 0, st>>>(b.N, (const double4 *) d_pos, (const double4 *) d_quat, b.orig, b.pinfo, b.bonds, b.d_sys,
 			b.rlist, b.pos, b.q64, b.q32, b.bpos, b.back64, b.d_state, b.any_rebuild, b.blist);
@@ -2968,9 +2998,10 @@ oxh_status oxh_batch_stats(oxh_batch *B, double *out6) {  // 12 doubles
 	return OXH_OK;
 }
 
-oxh_status oxh_batch_routes(oxh_batch *B, int *out1) {
-	if(!B || !out1) return fail(OXH_ERR_ARG, "bad arguments");
-	out1[0] = !B->persist && fused_ok(B);
+oxh_status oxh_batch_routes(oxh_batch *B, int *out2) {
+	if(!B || !out2) return fail(OXH_ERR_ARG, "bad arguments");
+	out2[0] = !B->persist && fused_ok(B);
+	out2[1] = B->b.far_lanes == 0 && !B->b.edge ? B->call_far_lanes : B->b.far_lanes;
 	return OXH_OK;
 }
 

@@ -98,3 +98,31 @@ def test_states_that_come_and_go(hip, monkeypatch, form):
                 assert vec_rel_err(add, want)[0] <= 10 * bar, (form, move)   # rounding of the additions onto O(1) values
             builds += move
             assert b.info()[0] == builds, (form, move)
+
+
+def test_far_kernel_of_calls_alone(hip):
+    """24 bundles of 960 nt with long rows (633 far pairs each): steps keep
+    the far pairs inline for the sake of one launch, force calls on the
+    caller's buffers take the far kernel, which is 6 % faster for them."""
+    from oracle import pyoracle as po
+    from oxdna_amd import systems
+    ss = [systems.duplex_bundle(2 + k, nx=4, ny=4, bp=30, spacing=2.6, lz=14.3, tc=30.0, salt=0.1) for k in range(24)]
+    n = sum(s.N for s in ss)
+    pos = np.zeros((n, 4))
+    pos[:, :3] = np.concatenate([s.pos for s in ss])
+    d_pos = DeviceArray(pos)
+    d_quat = DeviceArray(np.concatenate([hip.quat_from_frame(s.a1, s.a3) for s in ss]))
+    dF, dT = DeviceArray.zeros((n, 4), np.float32), DeviceArray.zeros((n, 4), np.float32)
+    with hip.HIPBatch(ss) as b:
+        before = b.stats()
+        assert b.routes()["call_far_lanes"] > 0
+        b.interaction_forces(d_pos.ptr, d_quat.ptr, dF.ptr, dT.ptr)
+        b.sync()
+        assert b.stats() == before
+    first = 0
+    for k, s in enumerate(ss):
+        if k in (0, 23):
+            ref = po.forces(po.Params(T=s.T, salt=s.salt), s)
+            assert vec_rel_err(dF.numpy()[first:first + s.N, :3].astype(np.float64), ref["F"])[0] <= 1e-5
+            assert vec_rel_err(dT.numpy()[first:first + s.N, :3].astype(np.float64), ref["T"])[0] <= 1e-5
+        first += s.N
