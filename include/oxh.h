@@ -173,20 +173,29 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *b, const double *d_pos, con
  * parameters and backend_precision from its keys; its pos, a1, a3, vel and
  * L are not read), with the state in d_pos / d_quat and the results added
  * onto d_forces / d_torques (layouts as above, particle k at index k).
- * Nothing is allocated: the Verlet list (built afresh on every call, all
- * pairs), the FP32 mirror, F, T and the parameters live in a fixed device
- * array of the library, OXH_NOALLOC_SCRATCH_BYTES on each GPU it runs on,
- * held until the process ends, and one page-locked host block that the
- * first call allocates.  Limits: at most OXH_NOALLOC_MAX_N
- * nucleotides (larger N is rejected with OXH_ERR_ARG before any GPU work)
- * and OXH_NOALLOC_MAX_NEIGH Verlet neighbours per nucleotide (more returns
- * OXH_ERR_SYSTEM and adds nothing).  The call queues its kernels on
- * `stream` (NULL: the null stream) and returns when they have run.  Every call on a GPU shares that GPU's array: calls that
- * overlap on one GPU (other threads, other streams, a call issued before
- * the previous call's additions have run) race; serialise them. */
+ * The call allocates nothing, on the device or the host: the Verlet list
+ * (built afresh on every call, all pairs), the FP32 mirror, F, T and the
+ * parameters live in a fixed device array of the library,
+ * OXH_NOALLOC_SCRATCH_BYTES on each GPU it runs on, held until the process
+ * ends.  Limits: at most OXH_NOALLOC_MAX_N nucleotides (larger N is rejected
+ * with OXH_ERR_ARG before any GPU work) and OXH_NOALLOC_MAX_NEIGH Verlet
+ * neighbours per nucleotide (more returns OXH_ERR_SYSTEM and adds nothing).
+ * The call queues its kernels on `stream` (NULL: the null stream) and
+ * returns when they have run, so it cannot be part of a capture of that
+ * stream.  Calls of one process share that array and are taken one after
+ * the other, whatever their threads and streams.
+ *
+ * oxh_noalloc_init(device) does what a first call would otherwise do, and
+ * allocates the one thing that makes calls faster: it has the library's code
+ * and device array loaded on that GPU, and takes one page-locked host block
+ * of 64 KB, the same for every GPU of the process, held until it ends.  To be
+ * called before serving or capturing starts; any number of times, from any
+ * thread.  Without it calls go through the library's static memory, with a
+ * copy each way. */
 #define OXH_NOALLOC_MAX_N 4096
 #define OXH_NOALLOC_MAX_NEIGH 256
-#define OXH_NOALLOC_SCRATCH_BYTES 5359872
+#define OXH_NOALLOC_SCRATCH_BYTES 5425408
+oxh_status oxh_noalloc_init(int device);
 oxh_status oxh_interaction_compute_forces_noalloc(int device, const oxh_system_desc *desc, const double *d_pos, const double *d_quat,
 		void *d_forces, void *d_torques, void *stream);
 

@@ -442,16 +442,31 @@ def philox(ctr: np.ndarray, key: np.ndarray, device: int = 0) -> np.ndarray:
     return out
 
 
+_noalloc_ready = set()
+
+
+def noalloc_init(device: int = 0):
+    """oxh_noalloc_init: loads what interaction_forces_noalloc needs on a
+    GPU, and allocates the page-locked block that makes it faster.  The first
+    call on that GPU does it too; to be called before that where nothing may
+    be allocated later (a serving loop, another thread's stream capture)."""
+    check(lib().oxh_noalloc_init(device), "oxh_noalloc_init")
+    _noalloc_ready.add(device)
+
+
 def interaction_forces_noalloc(system: System, d_pos: int, d_quat: int, d_forces: int, d_torques: int, stream: int = 0,
                                device: int = 0, **opts):
     """oxh_interaction_compute_forces_noalloc: adds the pair forces and
     torques of one system's state (caller device buffers, layouts as in
     HIPBatch.interaction_forces) to the caller's device buffers, with no
     device allocation (the library's fixed scratch array; at most
-    OXH_NOALLOC_MAX_N = 4096 nucleotides).  Topology and parameters come
+    OXH_NOALLOC_MAX_N = 4096 nucleotides), and on the host only its first
+    call on a GPU (noalloc_init).  Topology and parameters come
     from `system` and the options, as for HIPBatch; stream 0 is the null
     stream."""
     keep: list = []
     d = make_desc(system, keep, **opts)
+    if device not in _noalloc_ready and lib().oxh_noalloc_init(device) == 0:   # the call works without
+        _noalloc_ready.add(device)
     check(lib().oxh_interaction_compute_forces_noalloc(device, C.byref(d), d_pos, d_quat, d_forces, d_torques, stream or None),
           "oxh_interaction_compute_forces_noalloc")

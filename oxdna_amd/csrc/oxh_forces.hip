@@ -625,4 +625,9 @@ void launch_forces(hipStream_t st, const Batch &b, bool split, int k) {
 	launch_ext_forces(st, b, k);
 }
 
+hipError_t load_forces() {
+	hipFuncAttributes a;
+	return hipFuncGetAttributes(&a, (const void *) k_forces<8, false, true, true>);
+}
+
 }  // namespace oxh

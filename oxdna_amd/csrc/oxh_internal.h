@@ -248,6 +248,11 @@ void launch_export_state(const Batch &b, int first, int n, double *out);
 void launch_export_forces(const Batch &b, int first, int n, double *out);
 void launch_sums(const Batch &b, int n, int rows, const double *x, const double4 *vel, double *out);
 void launch_count(const Batch &b, long long *out);
+// loads a source file's kernels on the current device, as their first launch
+// would
+hipError_t load_forces();
+hipError_t load_lists();
+hipError_t load_rna();
 void launch_pair_quantities(hipStream_t st, const Batch &b, int sys, int kind, int n, const int4 *d_pairs, double *d_out);
 
 }  // namespace oxh

@@ -823,4 +823,9 @@ void launch_rna_forces(hipStream_t st, const Batch &b, bool split, int k) {
 	else rna::launch_lanes(st, b, b.F, b.T, split, k);
 }
 
+hipError_t load_rna() {
+	hipFuncAttributes a;
+	return hipFuncGetAttributes(&a, (const void *) rna::k_rna_pair_quantities);
+}
+
 }  // namespace oxh
