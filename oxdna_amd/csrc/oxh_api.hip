@@ -1212,7 +1212,7 @@ oxh_status autotune_forces(oxh_batch *B) {
 	const char *pack_env = getenv("OXH_PACK");
 	if(const char *env = getenv("OXH_FORCE_LANES")) {
 		b.lanes = atoi(env);
-		b.pack = !b.fp64 && b.lanes > 1 && pack_env && atoi(pack_env) == 1;
+		b.pack = !b.fp64 && !b.model && !B->persist && b.lanes > 1 && pack_env && atoi(pack_env) == 1;
 		if(const char *f = getenv("OXH_FAR_LANES")) b.far_lanes = atoi(f);
 		b.edge = b.ecap > 0 && edge_env && atoi(edge_env) == 1;
 		if(const char *g = getenv("OXH_EDGE_GROUP")) b.edge_group = atoi(g);
@@ -1814,15 +1814,17 @@ oxh_status create_impl(int device, int n_sys, const oxh_system_desc *descs, cons
 		if(s != OXH_OK) return bail(s);
 	}
 	else {
-		// the packed form: the bits of the in-place one, with HB, CRST and the
-		// bonds of a pool's few waves side by side (eight jobs of 259 to 1,332
-		// nt, a pass of 320 steps: 14.1 -> 13.0 ms)
-		b.pack = true;
-	}
-	if(const char *env = B->pool ? getenv("OXH_FORCE_LANES") : nullptr) {
-		b.lanes = atoi(env);
-		b.far_lanes = 0;
-		if(const char *f = getenv("OXH_FAR_LANES")) b.far_lanes = atoi(f);
+		if(const char *env = getenv("OXH_FORCE_LANES")) {
+			b.lanes = atoi(env);
+			b.far_lanes = 0;
+			if(const char *f = getenv("OXH_FAR_LANES")) b.far_lanes = atoi(f);
+		}
+		// the packed form: the bits of the in-place one (but with one lane per
+		// nucleotide), with HB, CRST and the bonds of a pool's few waves side
+		// by side (eight jobs of 259 to 1,332 nt, a pass of 320 steps: 14.1 ->
+		// 13.0 ms)
+		const char *e = getenv("OXH_PACK");
+		b.pack = !B->persist && b.lanes > 1 && !(e && atoi(e) == 0);
 	}
 	if(!fused_ok(B)) TRYB(free_step_buffers(B));
 	// graph chunk: enough steps to amortise the launch, at most ~2k kernels

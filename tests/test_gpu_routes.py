@@ -118,3 +118,39 @@ def test_second_buffers_only_while_steps_use_them(hip, monkeypatch):
         got = _final(b, 0)
     for key in KEYS:
         assert np.array_equal(want[key], got[key]), key
+
+
+@pytest.mark.parametrize("lanes", [None, 1, 2])
+def test_packed_form_of_pools(hip, monkeypatch, lanes):
+    """OXH_PACK=0 and one lane per nucleotide keep a pool in place; the bits are those of the packed form."""
+    jobs = [_gas(1, 30, 20), _gas(2, 3, 11), _gas(3, 9, 31)]
+    if lanes:
+        monkeypatch.setenv("OXH_FORCE_LANES", str(lanes))
+    got = []
+    for pack in (1, 0, None):
+        if pack is None:
+            monkeypatch.delenv("OXH_PACK")
+        else:
+            monkeypatch.setenv("OXH_PACK", str(pack))
+        with hip.HIPPool([2048] * 3) as p:
+            assert p.stats()["pack"] == (lanes != 1 and pack != 0)
+            for k, s in enumerate(jobs):
+                p.admit(k, s, 60 + 20 * k, seed=7 + k, dt=0.003, verlet_skin=0.05, refresh_vel=True, **THERMO["langevin"])
+            p.run(120)
+            got.append([_final(p, k) for k in range(3)])
+    _equal(got[0], got[1])
+    _equal(got[0], got[2])
+
+
+def test_packed_form_is_reported_only_where_there_is_one(hip, monkeypatch):
+    from test_gpu_rna import load_rna
+    monkeypatch.setenv("OXH_PACK", "1")
+    with hip.HIPPool([256] * 2) as p:   # workgroup engine
+        assert p.stats()["engine"] == "workgroup" and not p.stats()["pack"]
+    monkeypatch.setenv("OXH_FORCE_LANES", "4")
+    s, opts, _ = load_rna("rna_ff16_nohb")
+    with hip.HIPBatch(s, **opts) as b:
+        assert not b.stats()["pack"]
+    monkeypatch.setenv("OXH_PERSIST", "0")
+    with hip.HIPBatch(_gas(3, 30, 20), backend_precision="double") as b:
+        assert not b.stats()["pack"]
