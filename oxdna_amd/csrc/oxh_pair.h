@@ -22,13 +22,13 @@ namespace oxh {
 // the workgroup's particles (force, torque, energy), with four or more
 // lanes per nucleotide.  c: CXST results of each thread's pairs.  41 KB:
 // three workgroups per CU, as many as the registers allow.  Two entries per
-// lane and round (PACK_U = 2) measured slower (spilled registers and twice
-// the code): 242 against 237 us on the 196,608-nt bundle.
-constexpr int PACK_H = 22, PACK_U = 1, PACK_N = PACK_U * PACK_BS, PACK_BONDS = PACK_BS / 2;
+// lane and round measured slower (spilled registers and twice the code): 242
+// against 237 us on the 196,608-nt bundle.
+constexpr int PACK_H = 22, PACK_BONDS = PACK_BS / 2;
 struct PackShared {
-	float h[PACK_H][PACK_N];
-	float res[8][PACK_N];
-	float c[7][PACK_N];
+	float h[PACK_H][PACK_BS];
+	float res[8][PACK_BS];
+	float c[7][PACK_BS];
 	float bond[7][PACK_BONDS];
 	int n[2][2], rounds[PACK_BS / 64];
 };

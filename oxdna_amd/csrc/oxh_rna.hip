@@ -419,78 +419,74 @@ __device__ void nonbonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv
 	// hydrogen bonding (Watson-Crick-like pairs: base types summing to 3)
 	if(hb_open) {
 		const double rhmod = sqrt(rbmod2);
-		if((double) HYDR_RCLOW < rhmod && rhmod < (double) HYDR_RCHIGH) {
-			const dv3 rhdir = rbb * (1. / rhmod);
-			const double cost1 = -dot(a1, b1), cost2 = -dot(b1, rhdir), cost3 = dot(a1, rhdir);
-			const double cost4 = dot(a3, b3), cost7 = -dot(b3, rhdir), cost8 = dot(a3, rhdir);
-			const A t1 = lracos<A>(cost1), t2 = lracos<A>(cost2), t3 = lracos<A>(cost3);
-			const A t4 = lracos<A>(cost4), t7 = lracos<A>(cost7), t8 = lracos<A>(cost8);
-			const double ff1 = f1<0>(S, rhmod, q.type, p.type);
-			const double f4t1 = f4<HYDR_T1, A>(t1), f4t2 = f4<HYDR_T2, A>(t2), f4t3 = f4<HYDR_T3, A>(t3);
-			const double f4t4 = f4<HYDR_T4, A>(t4), f4t7 = f4<HYDR_T7, A>(t7), f4t8 = f4<HYDR_T8, A>(t8);
-			const double eh = ff1 * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8;
-			e[1] = eh;
-			if(eh != 0.) {
-				const double ff1D = f1D<0>(S, rhmod, q.type, p.type);
-				// d f4(acos c) / dc = -f4Dsin, with the signs the reference's
-				// mesh derivatives carry
-				const double f4t1Dsin = -f4Dsin<HYDR_T1, A>(t1, rsin<A>(cost1));
-				const double f4t2Dsin = -f4Dsin<HYDR_T2, A>(t2, rsin<A>(cost2));
-				const double f4t3Dsin = f4Dsin<HYDR_T3, A>(t3, rsin<A>(cost3));
-				const double f4t4Dsin = f4Dsin<HYDR_T4, A>(t4, rsin<A>(cost4));
-				const double f4t7Dsin = -f4Dsin<HYDR_T7, A>(t7, rsin<A>(cost7));
-				const double f4t8Dsin = f4Dsin<HYDR_T8, A>(t8, rsin<A>(cost8));
-				dv3 force = rhdir * (-ff1D * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8);
-				dv3 tl = cross(a3, b3) * (-(-ff1 * f4t1 * f4t2 * f4t3 * f4t4Dsin * f4t7 * f4t8));
-				tl -= cross(a1, b1) * (-ff1 * f4t1Dsin * f4t2 * f4t3 * f4t4 * f4t7 * f4t8);
-				force += (b1 + rhdir * cost2) * (1. / rhmod) * (ff1 * f4t1 * f4t2Dsin * f4t3 * f4t4 * f4t7 * f4t8);
-				force += (a1 - rhdir * cost3) * (1. / rhmod) * (ff1 * f4t1 * f4t2 * f4t3Dsin * f4t4 * f4t7 * f4t8);
-				tl += cross(rhdir, a1) * (-ff1 * f4t1 * f4t2 * f4t3Dsin * f4t4 * f4t7 * f4t8);
-				force += (b3 + rhdir * cost7) * (1. / rhmod) * (ff1 * f4t1 * f4t2 * f4t3 * f4t4 * f4t7Dsin * f4t8);
-				force += (a3 - rhdir * cost8) * (1. / rhmod) * (ff1 * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8Dsin);
-				tl += cross(rhdir, a3) * (-ff1 * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8Dsin);
-				fq += force;
-				tp += tl;
-				tp -= cross(pbase, force);
-			}
+		const dv3 rhdir = rbb * (1. / rhmod);
+		const double cost1 = -dot(a1, b1), cost2 = -dot(b1, rhdir), cost3 = dot(a1, rhdir);
+		const double cost4 = dot(a3, b3), cost7 = -dot(b3, rhdir), cost8 = dot(a3, rhdir);
+		const A t1 = lracos<A>(cost1), t2 = lracos<A>(cost2), t3 = lracos<A>(cost3);
+		const A t4 = lracos<A>(cost4), t7 = lracos<A>(cost7), t8 = lracos<A>(cost8);
+		const double ff1 = f1<0>(S, rhmod, q.type, p.type);
+		const double f4t1 = f4<HYDR_T1, A>(t1), f4t2 = f4<HYDR_T2, A>(t2), f4t3 = f4<HYDR_T3, A>(t3);
+		const double f4t4 = f4<HYDR_T4, A>(t4), f4t7 = f4<HYDR_T7, A>(t7), f4t8 = f4<HYDR_T8, A>(t8);
+		const double eh = ff1 * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8;
+		e[1] = eh;
+		if(eh != 0.) {
+			const double ff1D = f1D<0>(S, rhmod, q.type, p.type);
+			// d f4(acos c) / dc = -f4Dsin, with the signs the reference's
+			// mesh derivatives carry
+			const double f4t1Dsin = -f4Dsin<HYDR_T1, A>(t1, rsin<A>(cost1));
+			const double f4t2Dsin = -f4Dsin<HYDR_T2, A>(t2, rsin<A>(cost2));
+			const double f4t3Dsin = f4Dsin<HYDR_T3, A>(t3, rsin<A>(cost3));
+			const double f4t4Dsin = f4Dsin<HYDR_T4, A>(t4, rsin<A>(cost4));
+			const double f4t7Dsin = -f4Dsin<HYDR_T7, A>(t7, rsin<A>(cost7));
+			const double f4t8Dsin = f4Dsin<HYDR_T8, A>(t8, rsin<A>(cost8));
+			dv3 force = rhdir * (-ff1D * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8);
+			dv3 tl = cross(a3, b3) * (-(-ff1 * f4t1 * f4t2 * f4t3 * f4t4Dsin * f4t7 * f4t8));
+			tl -= cross(a1, b1) * (-ff1 * f4t1Dsin * f4t2 * f4t3 * f4t4 * f4t7 * f4t8);
+			force += (b1 + rhdir * cost2) * (1. / rhmod) * (ff1 * f4t1 * f4t2Dsin * f4t3 * f4t4 * f4t7 * f4t8);
+			force += (a1 - rhdir * cost3) * (1. / rhmod) * (ff1 * f4t1 * f4t2 * f4t3Dsin * f4t4 * f4t7 * f4t8);
+			tl += cross(rhdir, a1) * (-ff1 * f4t1 * f4t2 * f4t3Dsin * f4t4 * f4t7 * f4t8);
+			force += (b3 + rhdir * cost7) * (1. / rhmod) * (ff1 * f4t1 * f4t2 * f4t3 * f4t4 * f4t7Dsin * f4t8);
+			force += (a3 - rhdir * cost8) * (1. / rhmod) * (ff1 * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8Dsin);
+			tl += cross(rhdir, a3) * (-ff1 * f4t1 * f4t2 * f4t3 * f4t4 * f4t7 * f4t8Dsin);
+			fq += force;
+			tp += tl;
+			tp -= cross(pbase, force);
 		}
 	}
 
 	// cross stacking, on the base-base separation
 	if(cr_open) {
 		const double rcmod = sqrt(rbmod2);
-		if((double) F2_RCLOW[0] < rcmod && rcmod < (double) F2_RCHIGH[0]) {
-			const dv3 rcdir = rbb * (1. / rcmod);
-			const double cost2 = -dot(b1, rcdir), cost3 = dot(a1, rcdir), cost7 = -dot(b3, rcdir), cost8 = dot(a3, rcdir);
-			const double cost1 = -dot(a1, b1);
-			const A t1 = lracos<A>(cost1), t2 = lracos<A>(cost2), t3 = lracos<A>(cost3);
-			const A t7 = lracos<A>(cost7), t8 = lracos<A>(cost8);
-			const double ff2 = f2<0>(rcmod);
-			const double f4t1 = f4<CRST_T1, A>(t1), f4t2 = f4<CRST_T2, A>(t2), f4t3 = f4<CRST_T3, A>(t3);
-			const double f4t7 = f4<CRST_T7, A>(t7) + f4<CRST_T7, A>((A) PIf - t7);
-			const double f4t8 = f4<CRST_T8, A>(t8) + f4<CRST_T8, A>((A) PIf - t8);
-			const double ec = ff2 * f4t1 * f4t2 * f4t3 * f4t7 * f4t8;
-			e[2] = ec;
-			if(ec != 0.) {
-				const double ff2D = f2D<0>(rcmod);
-				const double f4t1Dsin = -f4Dsin<CRST_T1, A>(t1, rsin<A>(cost1));
-				const double f4t2Dsin = -f4Dsin<CRST_T2, A>(t2, rsin<A>(cost2));
-				const double f4t3Dsin = f4Dsin<CRST_T3, A>(t3, rsin<A>(cost3));
-				const double f4t7Dsin = -f4Dsin<CRST_T7, A>(t7, rsin<A>(cost7)) + f4Dsin<CRST_T7, A>((A) PIf - t7, rsin_pi<1, A>(cost7));
-				const double f4t8Dsin = f4Dsin<CRST_T8, A>(t8, rsin<A>(cost8)) - f4Dsin<CRST_T8, A>((A) PIf - t8, rsin_pi<1, A>(cost8));
-				// the reference's theta4 factor is 1 here, its derivative 0
-				dv3 force = rcdir * (-(ff2D * f4t1 * f4t2 * f4t3 * f4t7 * f4t8));
-				dv3 tl = cross(a1, b1) * (-(-ff2 * f4t1Dsin * f4t2 * f4t3 * f4t7 * f4t8));
-				force += (b1 + rcdir * cost2) * (ff2 * f4t1 * f4t2Dsin * f4t3 * f4t7 * f4t8 / rcmod);
-				force += (a1 - rcdir * cost3) * (ff2 * f4t1 * f4t2 * f4t3Dsin * f4t7 * f4t8 / rcmod);
-				tl += cross(rcdir, a1) * (-ff2 * f4t1 * f4t2 * f4t3Dsin * f4t7 * f4t8);
-				force += (b3 + rcdir * cost7) * (1. / rcmod) * (ff2 * f4t1 * f4t2 * f4t3 * f4t7Dsin * f4t8);
-				force += (a3 - rcdir * cost8) * (1. / rcmod) * (ff2 * f4t1 * f4t2 * f4t3 * f4t7 * f4t8Dsin);
-				tl += cross(rcdir, a3) * (-ff2 * f4t1 * f4t2 * f4t3 * f4t7 * f4t8Dsin);
-				fq += force;
-				tp += tl;
-				tp -= cross(pbase, force);
-			}
+		const dv3 rcdir = rbb * (1. / rcmod);
+		const double cost2 = -dot(b1, rcdir), cost3 = dot(a1, rcdir), cost7 = -dot(b3, rcdir), cost8 = dot(a3, rcdir);
+		const double cost1 = -dot(a1, b1);
+		const A t1 = lracos<A>(cost1), t2 = lracos<A>(cost2), t3 = lracos<A>(cost3);
+		const A t7 = lracos<A>(cost7), t8 = lracos<A>(cost8);
+		const double ff2 = f2<0>(rcmod);
+		const double f4t1 = f4<CRST_T1, A>(t1), f4t2 = f4<CRST_T2, A>(t2), f4t3 = f4<CRST_T3, A>(t3);
+		const double f4t7 = f4<CRST_T7, A>(t7) + f4<CRST_T7, A>((A) PIf - t7);
+		const double f4t8 = f4<CRST_T8, A>(t8) + f4<CRST_T8, A>((A) PIf - t8);
+		const double ec = ff2 * f4t1 * f4t2 * f4t3 * f4t7 * f4t8;
+		e[2] = ec;
+		if(ec != 0.) {
+			const double ff2D = f2D<0>(rcmod);
+			const double f4t1Dsin = -f4Dsin<CRST_T1, A>(t1, rsin<A>(cost1));
+			const double f4t2Dsin = -f4Dsin<CRST_T2, A>(t2, rsin<A>(cost2));
+			const double f4t3Dsin = f4Dsin<CRST_T3, A>(t3, rsin<A>(cost3));
+			const double f4t7Dsin = -f4Dsin<CRST_T7, A>(t7, rsin<A>(cost7)) + f4Dsin<CRST_T7, A>((A) PIf - t7, rsin_pi<1, A>(cost7));
+			const double f4t8Dsin = f4Dsin<CRST_T8, A>(t8, rsin<A>(cost8)) - f4Dsin<CRST_T8, A>((A) PIf - t8, rsin_pi<1, A>(cost8));
+			// the reference's theta4 factor is 1 here, its derivative 0
+			dv3 force = rcdir * (-(ff2D * f4t1 * f4t2 * f4t3 * f4t7 * f4t8));
+			dv3 tl = cross(a1, b1) * (-(-ff2 * f4t1Dsin * f4t2 * f4t3 * f4t7 * f4t8));
+			force += (b1 + rcdir * cost2) * (ff2 * f4t1 * f4t2Dsin * f4t3 * f4t7 * f4t8 / rcmod);
+			force += (a1 - rcdir * cost3) * (ff2 * f4t1 * f4t2 * f4t3Dsin * f4t7 * f4t8 / rcmod);
+			tl += cross(rcdir, a1) * (-ff2 * f4t1 * f4t2 * f4t3Dsin * f4t7 * f4t8);
+			force += (b3 + rcdir * cost7) * (1. / rcmod) * (ff2 * f4t1 * f4t2 * f4t3 * f4t7Dsin * f4t8);
+			force += (a3 - rcdir * cost8) * (1. / rcmod) * (ff2 * f4t1 * f4t2 * f4t3 * f4t7 * f4t8Dsin);
+			tl += cross(rcdir, a3) * (-ff2 * f4t1 * f4t2 * f4t3 * f4t7 * f4t8Dsin);
+			fq += force;
+			tp += tl;
+			tp -= cross(pbase, force);
 		}
 	}
 
@@ -507,75 +503,73 @@ __device__ void nonbonded(const oxh_sys &S, const Nuc &p, const Nuc &q, const dv
 	}
 	if(cx_open) {
 		const double rsmod = sqrt(rs2);
-		if((double) F2_RCLOW[1] < rsmod && rsmod < (double) F2_RCHIGH[1]) {
-			const dv3 rsdir = rstack * (1. / rsmod);
-			const double cost5 = dot(a3, rsdir), cost6 = -dot(b3, rsdir);
-			const double cost1 = -dot(a1, b1), cost4 = dot(a3, b3);
-			const A t1 = lracos<A>(cost1), t4 = lracos<A>(cost4), t5 = lracos<A>(cost5), t6 = lracos<A>(cost6);
-			const double rbmod = sqrt(dot(rback, rback));
-			const dv3 rbdir = rback * (1. / rbmod);
-			const double cosphi3 = dot(rsdir, cross(rbdir, a1));
-			const double cosphi4 = dot(rsdir, cross(rbdir, b1));
-			const double ff2 = f2<1>(rsmod);
-			const A t1b = (A) (2 * PIf) - t1;
-			const double f4t1 = f4<CXST_T1, A>(t1) + f4<CXST_T1, A>(t1b);
-			const double f4t4 = f4<CXST_T4, A>(t4);
-			const double f4t5 = f4<CXST_T5, A>(t5) + f4<CXST_T5, A>((A) PIf - t5);
-			const double f4t6 = f4<CXST_T6, A>(t6) + f4<CXST_T6, A>((A) PIf - t6);
-			const double f5c3 = f5<CXST_PHI3>(cosphi3);
-			const double f5c4 = f5<CXST_PHI4>(cosphi4);
-			const double ecx = ff2 * f4t1 * f4t4 * f4t5 * f4t6 * f5c3 * f5c4;
-			e[3] = ecx;
-			if(ecx != 0.) {
-				const double ff2D = f2D<1>(rsmod);
-				const double f4t1Dsin = -f4Dsin<CXST_T1, A>(t1, rsin<A>(cost1)) + f4Dsin<CXST_T1, A>(t1b, -rsin_pi<2, A>(cost1));
-				const double f4t4Dsin = f4Dsin<CXST_T4, A>(t4, rsin<A>(cost4));
-				const double f4t5Dsin = f4Dsin<CXST_T5, A>(t5, rsin<A>(cost5)) - f4Dsin<CXST_T5, A>((A) PIf - t5, rsin_pi<1, A>(cost5));
-				const double f4t6Dsin = -f4Dsin<CXST_T6, A>(t6, rsin<A>(cost6)) + f4Dsin<CXST_T6, A>((A) PIf - t6, rsin_pi<1, A>(cost6));
-				const double f5Dc3 = f5D<CXST_PHI3>(cosphi3);
-				const double f5Dc4 = f5D<CXST_PHI4>(cosphi4);
-				dv3 force = rsdir * (-ff2D * f4t1 * f4t4 * f4t5 * f4t6 * f5c3 * f5c4);
-				dv3 tl = cross(a1, b1) * (-(-ff2 * f4t1Dsin * f4t4 * f4t5 * f4t6 * f5c3 * f5c4));
-				tl -= cross(a3, b3) * (-ff2 * f4t1 * f4t4Dsin * f4t5 * f4t6 * f5c3 * f5c4);
-				const double fact5 = ff2 * f4t1 * f4t4 * f4t5Dsin * f4t6 * f5c3 * f5c4;
-				force += (a3 - rsdir * cost5) * (fact5 / rsmod);
-				tl -= cross(rsdir, a3) * fact5;
-				const double fact6 = ff2 * f4t1 * f4t4 * f4t5 * f4t6Dsin * f5c3 * f5c4;
-				force += (b3 + rsdir * cost6) * (1. / rsmod) * fact6;
-				tl -= cross(pst, force);
+		const dv3 rsdir = rstack * (1. / rsmod);
+		const double cost5 = dot(a3, rsdir), cost6 = -dot(b3, rsdir);
+		const double cost1 = -dot(a1, b1), cost4 = dot(a3, b3);
+		const A t1 = lracos<A>(cost1), t4 = lracos<A>(cost4), t5 = lracos<A>(cost5), t6 = lracos<A>(cost6);
+		const double rbmod = sqrt(dot(rback, rback));
+		const dv3 rbdir = rback * (1. / rbmod);
+		const double cosphi3 = dot(rsdir, cross(rbdir, a1));
+		const double cosphi4 = dot(rsdir, cross(rbdir, b1));
+		const double ff2 = f2<1>(rsmod);
+		const A t1b = (A) (2 * PIf) - t1;
+		const double f4t1 = f4<CXST_T1, A>(t1) + f4<CXST_T1, A>(t1b);
+		const double f4t4 = f4<CXST_T4, A>(t4);
+		const double f4t5 = f4<CXST_T5, A>(t5) + f4<CXST_T5, A>((A) PIf - t5);
+		const double f4t6 = f4<CXST_T6, A>(t6) + f4<CXST_T6, A>((A) PIf - t6);
+		const double f5c3 = f5<CXST_PHI3>(cosphi3);
+		const double f5c4 = f5<CXST_PHI4>(cosphi4);
+		const double ecx = ff2 * f4t1 * f4t4 * f4t5 * f4t6 * f5c3 * f5c4;
+		e[3] = ecx;
+		if(ecx != 0.) {
+			const double ff2D = f2D<1>(rsmod);
+			const double f4t1Dsin = -f4Dsin<CXST_T1, A>(t1, rsin<A>(cost1)) + f4Dsin<CXST_T1, A>(t1b, -rsin_pi<2, A>(cost1));
+			const double f4t4Dsin = f4Dsin<CXST_T4, A>(t4, rsin<A>(cost4));
+			const double f4t5Dsin = f4Dsin<CXST_T5, A>(t5, rsin<A>(cost5)) - f4Dsin<CXST_T5, A>((A) PIf - t5, rsin_pi<1, A>(cost5));
+			const double f4t6Dsin = -f4Dsin<CXST_T6, A>(t6, rsin<A>(cost6)) + f4Dsin<CXST_T6, A>((A) PIf - t6, rsin_pi<1, A>(cost6));
+			const double f5Dc3 = f5D<CXST_PHI3>(cosphi3);
+			const double f5Dc4 = f5D<CXST_PHI4>(cosphi4);
+			dv3 force = rsdir * (-ff2D * f4t1 * f4t4 * f4t5 * f4t6 * f5c3 * f5c4);
+			dv3 tl = cross(a1, b1) * (-(-ff2 * f4t1Dsin * f4t4 * f4t5 * f4t6 * f5c3 * f5c4));
+			tl -= cross(a3, b3) * (-ff2 * f4t1 * f4t4Dsin * f4t5 * f4t6 * f5c3 * f5c4);
+			const double fact5 = ff2 * f4t1 * f4t4 * f4t5Dsin * f4t6 * f5c3 * f5c4;
+			force += (a3 - rsdir * cost5) * (fact5 / rsmod);
+			tl -= cross(rsdir, a3) * fact5;
+			const double fact6 = ff2 * f4t1 * f4t4 * f4t5 * f4t6Dsin * f5c3 * f5c4;
+			force += (b3 + rsdir * cost6) * (1. / rsmod) * fact6;
+			tl -= cross(pst, force);
 
-				// phi3 (on a1) and phi4 (on b1): forces on the stack and
-				// backbone sites, torques on p as the reference collects them
-				double force_c = ff2 * f4t1 * f4t4 * f4t5 * f4t6 * f5c4 * f5Dc3;
-				dv3 rba1 = cross(rbdir, a1);
-				dv3 a1rs = cross(a1, rsdir);
-				double rb_dot_a1rs = dot(rbdir, a1rs);
-				double rs_dot_rba1 = dot(rsdir, rba1);
-				dv3 fst = (rba1 - rsdir * rs_dot_rba1) * (-(force_c / rsmod));
-				dv3 fbk = (a1rs - rbdir * rb_dot_a1rs) * (-(force_c / rbmod));
-				dv3 myforce = fst;
-				myforce += fbk;
-				dv3 mt1 = -cross(pst, fst);
-				mt1 -= cross(pback, fbk);
-				mt1 -= cross(a1, cross(rsdir, rbdir)) * force_c;
+			// phi3 (on a1) and phi4 (on b1): forces on the stack and
+			// backbone sites, torques on p as the reference collects them
+			double force_c = ff2 * f4t1 * f4t4 * f4t5 * f4t6 * f5c4 * f5Dc3;
+			dv3 rba1 = cross(rbdir, a1);
+			dv3 a1rs = cross(a1, rsdir);
+			double rb_dot_a1rs = dot(rbdir, a1rs);
+			double rs_dot_rba1 = dot(rsdir, rba1);
+			dv3 fst = (rba1 - rsdir * rs_dot_rba1) * (-(force_c / rsmod));
+			dv3 fbk = (a1rs - rbdir * rb_dot_a1rs) * (-(force_c / rbmod));
+			dv3 myforce = fst;
+			myforce += fbk;
+			dv3 mt1 = -cross(pst, fst);
+			mt1 -= cross(pback, fbk);
+			mt1 -= cross(a1, cross(rsdir, rbdir)) * force_c;
 
-				force_c = ff2 * f4t1 * f4t4 * f4t5 * f4t6 * f5c3 * f5Dc4;
-				rba1 = cross(rbdir, b1);
-				a1rs = cross(b1, rsdir);
-				rb_dot_a1rs = dot(rbdir, a1rs);
-				rs_dot_rba1 = dot(rsdir, rba1);
-				fst = (rba1 - rsdir * rs_dot_rba1) * (-(force_c / rsmod));
-				fbk = (a1rs - rbdir * rb_dot_a1rs) * (-(force_c / rbmod));
-				myforce += fst;
-				myforce += fbk;
-				mt1 -= cross(pst, fst);
-				mt1 -= cross(pback, fbk);
+			force_c = ff2 * f4t1 * f4t4 * f4t5 * f4t6 * f5c3 * f5Dc4;
+			rba1 = cross(rbdir, b1);
+			a1rs = cross(b1, rsdir);
+			rb_dot_a1rs = dot(rbdir, a1rs);
+			rs_dot_rba1 = dot(rsdir, rba1);
+			fst = (rba1 - rsdir * rs_dot_rba1) * (-(force_c / rsmod));
+			fbk = (a1rs - rbdir * rb_dot_a1rs) * (-(force_c / rbmod));
+			myforce += fst;
+			myforce += fbk;
+			mt1 -= cross(pst, fst);
+			mt1 -= cross(pback, fbk);
 
-				force += myforce;
-				tl += mt1;
-				fq += force;
-				tp += tl;
-			}
+			force += myforce;
+			tl += mt1;
+			fq += force;
+			tp += tl;
 		}
 	}
 }
