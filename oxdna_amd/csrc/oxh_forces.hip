@@ -261,15 +261,15 @@ __global__ void __launch_bounds__(256) k_forces_far(int N, const double4 *__rest
 		int xcd) {
 	const int blk = xcd ? xcd_block(((unsigned) N * K + blockDim.x - 1) / blockDim.x) : (int) blockIdx.x;
 	if(blk < 0) return;
-	if(k_step == K_IF_LISTS_HOLD && *any) return;
+	const int hold = k_step == K_IF_LISTS_HOLD ? *any : 0;
 	const int t = blk * blockDim.x + threadIdx.x;
 	const int i = t / K;
 	const int l = t % K;
 	if(i >= N) return;
 	const int s = pinfo[i].y;
 	const oxh_sys &S = systems[s];
-	if(idle(i, S, s, k_step, limit)) return;
 	const int nf = nnbr[i].y;
+	if(hold || idle(i, S, s, k_step, limit)) return;
 	const int *row = nbr + (size_t) i * max_neigh + max_neigh - 1;
 	const float4 Bi = bpos[i];
 	f3 Ff = {0, 0, 0};
@@ -378,15 +378,15 @@ __global__ void __launch_bounds__(256) k_forces_far_dp(int N, const double4 *__r
 		int xcd) {
 	const int blk = xcd ? xcd_block(((unsigned) N * K + blockDim.x - 1) / blockDim.x) : (int) blockIdx.x;
 	if(blk < 0) return;
-	if(k_step == K_IF_LISTS_HOLD && *any) return;
+	const int hold = k_step == K_IF_LISTS_HOLD ? *any : 0;
 	const int t = blk * blockDim.x + threadIdx.x;
 	const int i = t / K;
 	const int l = t % K;
 	if(i >= N) return;
 	const int s = pinfo[i].y;
 	const oxh_sys &S = systems[s];
-	if(idle(i, S, s, k_step, limit)) return;
 	const int nf = nnbr[i].y;
+	if(hold || idle(i, S, s, k_step, limit)) return;
 	const int *row = nbr + (size_t) i * max_neigh + max_neigh - 1;
 	const double4 Pi = pos[i];
 	Sites64 si;
