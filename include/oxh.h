@@ -216,7 +216,8 @@ oxh_status oxh_batch_hilbert_sort(oxh_batch *b);
  * velocities, angular momenta and quaternions, the positions of the last
  * list build, the forces of the current state, the per-particle RNG step
  * counters, the particle order, Bussi's internal kinetic energies, the step
- * counters and the force launch shape -- as one opaque byte buffer.
+ * counters, the launch shape and the form of the step's kernels (packed or
+ * in place, one launch per step or one per phase) -- as one opaque buffer.
  * Restored into a batch created from the same systems (same descs), the
  * run continues bitwise as if it had not been interrupted: the lists are
  * rebuilt exactly from their build positions and the Philox streams
@@ -477,8 +478,8 @@ oxh_status oxh_batch_set_state(oxh_batch *b, int sys, const double *pos, const d
  * has at most 512 nucleotides and no cells, 2: one kernel per phase with
  * the close pairs in half-list form, each pair evaluated once -- the
  * reference's use_edge), out[9] number of systems, out[10] 1 when the
- * close kernel takes the packed form (HB, cross and coaxial stacking of a
- * workgroup's close pairs evaluated from work lists in LDS, one pair per
+ * close kernel takes the packed form (HB and cross stacking of a
+ * workgroup's close pairs evaluated from a work list in LDS, one pair per
  * thread; same results bit for bit), else 0, out[11] number of systems
  * whose far pairs are kept by their backbone sites (far pairs then enter
  * the list only while their backbone sites are within the Debye-Hueckel

@@ -21,8 +21,9 @@
 // index) by ranking its entries, so rows and forces are those of the other
 // path.  Rows above STEP_ROW entries have a launch of their own before the
 // step's, for the systems that have met one.
-// Measured, per MD step: 24,576-nt gas with Bussi 39 -> 35 us, 777 nt without
-// cells 20 -> 17 us, a pool of eight jobs of 259 to 1,332 nt 44 -> 41 us.
+// Measured, per MD step, one kernel per phase -> this: 24,576-nt gas with
+// Bussi 36.5 -> 33.2 us, 777 nt without cells 16.5 -> 13.0 us, a pool of eight
+// jobs of 259 to 1,332 nt 43.6 -> 37.9 us.
 // Not for dense batches (their lists are built cell by cell), far pairs in a
 // kernel of their own, the half-list form, all-FP64, oxRNA or external
 // forces, which keep the one-kernel-per-phase path.
