@@ -167,8 +167,8 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *b, const double *d_pos, con
 		void *stream);
 
 /* No counterpart in the reference.  For callers that cannot allocate device
- * memory (code under HIP graph capture, serving loops, harnesses that forbid
- * hipMalloc): the same additions as oxh_interaction_compute_forces, for ONE
+ * memory (serving loops, programs that take theirs at the start, harnesses
+ * that forbid hipMalloc): the same additions as oxh_interaction_compute_forces, for ONE
  * system described by desc (topology from its btype / n3 / n5 host arrays,
  * parameters and backend_precision from its keys; its pos, a1, a3, vel and
  * L are not read), with the state in d_pos / d_quat and the results added
@@ -189,8 +189,8 @@ oxh_status oxh_interaction_compute_forces(oxh_batch *b, const double *d_pos, con
  * allocates the one thing that makes calls faster: it has the library's code
  * and device array loaded on that GPU, and takes one page-locked host block
  * of 64 KB, the same for every GPU of the process, held until it ends.  To be
- * called before serving or capturing starts; any number of times, from any
- * thread.  Without it calls go through the library's static memory, with a
+ * called before serving starts, and while no thread captures a stream; any
+ * number of times, from any thread.  Without it calls go through the library's static memory, with a
  * copy each way. */
 #define OXH_NOALLOC_MAX_N 4096
 #define OXH_NOALLOC_MAX_NEIGH 256

@@ -449,7 +449,7 @@ def noalloc_init(device: int = 0):
     """oxh_noalloc_init: loads what interaction_forces_noalloc needs on a
     GPU, and allocates the page-locked block that makes it faster.  The first
     call on that GPU does it too; to be called before that where nothing may
-    be allocated later (a serving loop, another thread's stream capture)."""
+    be allocated later."""
     check(lib().oxh_noalloc_init(device), "oxh_noalloc_init")
     _noalloc_ready.add(device)
 

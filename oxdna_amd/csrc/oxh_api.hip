@@ -3129,6 +3129,10 @@ oxh_status oxh_batch_restore(oxh_batch *B, const void *buf, size_t bytes) {
 		return fail(OXH_ERR_ARG, "checkpoint of systems with other sizes, boxes or parameters than this batch's");
 	HIPCHK(hipSetDevice(b.device));
 	HIPCHK(hipStreamSynchronize(b.stream));
+	if(b.graph_exec) {
+		(void) hipGraphExecDestroy(b.graph_exec);
+		b.graph_exec = nullptr;
+	}
 	// the checkpointed launch shape, so that forces round as they did
 	if(h.edge && b.ecap == 0) TRY(alloc_edges(B, h.ecap > 0 ? h.ecap : std::min(b.max_neigh, 64)));
 	if(!h.edge && b.ecap > 0) TRY(alloc_edges(B, 0));
@@ -3141,8 +3145,8 @@ oxh_status oxh_batch_restore(oxh_batch *B, const void *buf, size_t bytes) {
 	if(h.form & CKPT_FORM) {
 		b.pack = (h.form & CKPT_PACK) != 0;
 		b.fuse = (h.form & CKPT_FUSE) != 0 && can_fuse(B);
-		if(fused_ok(B)) TRY(alloc_step_buffers(B));
 	}
+	TRY(fused_ok(B) ? alloc_step_buffers(B) : free_step_buffers(B));
 	const char *p = (const char *) buf + sizeof(h);
 	for(auto &x : ckpt_layout(B)) {
 		HIPCHK(hipMemcpyAsync(x.first, p, x.second, hipMemcpyHostToDevice, b.stream));
@@ -3152,10 +3156,6 @@ oxh_status oxh_batch_restore(oxh_batch *B, const void *buf, size_t bytes) {
 	b.step = h.step;
 	B->since_sort = h.since_sort;
 	B->since_fix = h.since_fix;
-	if(b.graph_exec) {
-		(void) hipGraphExecDestroy(b.graph_exec);
-		b.graph_exec = nullptr;
-	}
 	oxh::launch_prepare_mirror(b.stream, b);
 	oxh::launch_slot_of(b.stream, b);
 	// the lists of the checkpointed run, rebuilt exactly from their build
